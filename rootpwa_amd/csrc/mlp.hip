@@ -1,10 +1,12 @@
 // mlp.hip -- the learned initializer's network (include/rootpwa_amd_mlp.h).
 //
-// Products run on FP32 MFMA (v_mfma_f32_32x32x2f32, one 32x32 output tile per
-// wave, operands straight from global memory: the matrices are small and stay
-// in L2); bias, GELU, loss and Adam are elementwise kernels.  Every reduction
-// (the K loop of a product, the bias gradients, the loss) runs in a fixed
-// order, so training is deterministic for a given seed.
+// Products run on FP32 MFMA (v_mfma_f32_16x16x4_f32) with everything that is
+// elementwise fused into them: bias, GELU, the loss and its gradient, GELU', the
+// bias gradients and Adam.  A training step of L layers is 2 L launches: L
+// forward products, L - 1 products dZ W^T, and one launch for the weight
+// gradients and the Adam update of all layers.  Every reduction (the K split of
+// a product, the sum over a batch's rows, the loss) runs in a fixed order, so
+// training is deterministic for a given seed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,8 +22,6 @@
 namespace rpwa_amd {
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 constexpr float kInvSqrt2 = 0.70710678118654752440f;
 constexpr float kInvSqrt2Pi = 0.39894228040143267794f;
 
@@ -32,118 +32,286 @@ __device__ __forceinline__ float gelu_grad(float z)
 	return 0.5f * (1.f + erff(z * kInvSqrt2)) + z * kInvSqrt2Pi * expf(-0.5f * z * z);
 }
 
-enum Epilogue { EPI_STORE = 0, EPI_BIAS_GELU = 1, EPI_BIAS = 2 };
+// What bounds a product here: latency.  At the training batch of 64 rows the
+// largest one is 64 x 512 x 775 (51 MFLOP, 1.6 MB of weights out of L2): one
+// 32 x 32 tile per wave gave 64 waves, each a chain of 388 dependent load /
+// MFMA steps (111 us).  So a workgroup owns one 16 x 16 tile (128 workgroups
+// there) and its kGemmWaves waves split K: wave w takes the 16-deep K groups w,
+// w + 8, ..., kGemmDeep of them loaded before the first MFMA, and the waves'
+// sums are added in wave order through LDS (5.0 us on average over the hidden
+// layers; a training step of the 775 - 3 x 512 - 176 network 730 -> 50 us).
+constexpr int kGemmWaves = 8;
+constexpr int kGemmThreads = 64 * kGemmWaves;
+constexpr int kGemmDeep = 4;  // 16-deep K groups in flight per wave
 
-// C[M][N] = op(A) op(B) (+ epilogue); op(A)(m, k) = TA ? A[k lda + m] : A[m lda + k],
-// op(B)(k, n) = TB ? B[n ldb + k] : B[k ldb + n].  Block: 4 waves, 64 x 64 tile.
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void gemm_kernel(const float* __restrict__ A, int lda, const float* __restrict__ B,
-                                                   int ldb, float* __restrict__ C, int ldc, int M, int N, int K,
-                                                   const float* __restrict__ bias, float* __restrict__ H)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+enum Epilogue {
+	EPI_HIDDEN = 0,  // Z = s + bias, H = GELU(Z)
+	EPI_OUT = 1,     // Z = s + bias
+	EPI_LOSS = 2,    // Z = s + bias, dZ = 2 (Z - T) / n, the tile's sum of (Z - T)^2
+	EPI_DZ = 3       // dZ = s GELU'(Z)
+};
+
+struct GemmArgs {
+	const float* A;         // [M][lda], row r at A + (rowIdx ? rowIdx[r] : r) lda
+	const uint32_t* rowIdx;
+	const float* B;         // TB ? [N][ldb] : [K][ldb]
+	int lda, ldb, M, N, K;
+	const float* bias;      // [N]
+	float* Z;               // [M][N] pre-activations (written, or read by EPI_DZ)
+	float* out;             // [M][N] H (EPI_HIDDEN) or dZ (EPI_LOSS, EPI_DZ)
+	const float* T;         // targets [.][N], row i at T + (tIdx ? tIdx[i] : i) N
+	const uint32_t* tIdx;
+	float scale;            // 2 / (M N)
+	double* tileLoss;       // per workgroup
+};
+
+// 4 consecutive floats at p (aligned to 4 bytes only: rows of any length), zero past `left`
+__device__ __forceinline__ f32x4 load4(const float* p, int left)
 {
-	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-	const int m0 = blockIdx.y * 64 + 32 * (wave >> 1), n0 = blockIdx.x * 64 + 32 * (wave & 1);
-	const int r = lane & 31, kk = lane >> 5;
-	const int am = m0 + r, bn = n0 + r;
-	f32x16 acc = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-	for (int k = 0; k < K; k += 2) {
-		const int ka = k + kk;
-		float a = 0.f, b = 0.f;
-		if (am < M && ka < K)
-			a = TA ? A[(size_t)ka * lda + am] : A[(size_t)am * lda + ka];
-		if (bn < N && ka < K)
-			b = TB ? B[(size_t)bn * ldb + ka] : B[(size_t)ka * ldb + bn];
-		acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+	f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+	if (left >= 4)
+		__builtin_memcpy(&v, p, 16);
+	else {
+		if (left > 0)
+			v.x = p[0];
+		if (left > 1)
+			v.y = p[1];
+		if (left > 2)
+			v.z = p[2];
 	}
-	// D[i][j]: column j = lane % 32, row i = 8 (v / 4) + 4 (lane / 32) + v % 4
+	return v;
+}
+
+// the first `left` of v's values to p
+__device__ __forceinline__ void store4(float* p, const f32x4 v, int left)
+{
+	if (left >= 4)
+		__builtin_memcpy(p, &v, 16);
+	else {
+		if (left > 0)
+			p[0] = v.x;
+		if (left > 1)
+			p[1] = v.y;
+		if (left > 2)
+			p[2] = v.z;
+	}
+}
+
+// C = A op(B) on one 16 x 16 tile.  MFMA i of a K group takes k = 16 g + 4 q + i
+// in lane quarter q (lane / 16), so a lane's four values are consecutive in a row.
+template <bool TB, int EPI>
+__global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs a)
+{
+	__shared__ float red[kGemmWaves][256];
+	__shared__ double sq[256];
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+	const int r = lane & 15, q = lane >> 4;
+	const uint32_t nx = ((uint32_t)a.N + 15) / 16;
+	const int m0 = (int)(blockIdx.x / nx) * 16, n0 = (int)(blockIdx.x % nx) * 16;
+	const int m = m0 + r, n = n0 + r;
+	// rows and columns past the edge repeat the last one; their outputs are not stored
+	const int mc = min(m, a.M - 1), nc = min(n, a.N - 1);
+	const float* pa = a.A + (size_t)(a.rowIdx ? a.rowIdx[mc] : (uint32_t)mc) * a.lda;
+	const float* pb = TB ? a.B + (size_t)nc * a.ldb : a.B + nc;
+	const int groups = (a.K + 15) / 16;
+	f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+	for (int g0 = wave; g0 < groups; g0 += kGemmWaves * kGemmDeep) {
+		f32x4 av[kGemmDeep], bv[kGemmDeep];
 #pragma unroll
-	for (int v = 0; v < 16; ++v) {
-		const int i = m0 + 8 * (v >> 2) + 4 * kk + (v & 3), jn = n0 + r;
-		if (i < M && jn < N) {
-			float z = acc[v];
-			if (EPI != EPI_STORE)
-				z += bias[jn];
-			C[(size_t)i * ldc + jn] = z;
-			if (EPI == EPI_BIAS_GELU)
-				H[(size_t)i * ldc + jn] = gelu(z);
+		for (int d = 0; d < kGemmDeep; ++d) {
+			const int g = g0 + d * kGemmWaves, k = 16 * g + 4 * q;
+			if (16 * g + 16 <= a.K) {  // the same in every lane
+				av[d] = load4(pa + k, 4);
+				if (TB)
+					bv[d] = load4(pb + k, 4);
+				else
+#pragma unroll
+					for (int i = 0; i < 4; ++i)
+						bv[d][i] = pb[(size_t)(k + i) * a.ldb];
+			} else {  // the last, partial group, and none
+				const int left = a.K - k;
+				av[d] = load4(pa + k, left);
+				if (TB)
+					bv[d] = load4(pb + k, left);
+				else
+#pragma unroll
+					for (int i = 0; i < 4; ++i)
+						bv[d][i] = i < left ? pb[(size_t)(k + i) * a.ldb] : 0.f;
+			}
+		}
+#pragma unroll
+		for (int d = 0; d < kGemmDeep; ++d)
+#pragma unroll
+			for (int i = 0; i < 4; ++i)
+				acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[d][i], bv[d][i], acc, 0, 0, 0);
+	}
+	// D[i][j]: column j = lane % 16, row i = 4 (lane / 16) + register
+#pragma unroll
+	for (int v = 0; v < 4; ++v)
+		red[wave][(4 * q + v) * 16 + r] = acc[v];
+	__syncthreads();
+	const int t = threadIdx.x;
+	double d2 = 0.;
+	if (t < 256) {
+		float s = red[0][t];
+#pragma unroll
+		for (int w = 1; w < kGemmWaves; ++w)
+			s += red[w][t];
+		const int i = m0 + t / 16, j = n0 + t % 16;
+		if (i < a.M && j < a.N) {
+			const size_t o = (size_t)i * a.N + j;
+			if (EPI == EPI_DZ) {
+				a.out[o] = s * gelu_grad(a.Z[o]);
+			} else {
+				const float z = s + a.bias[j];
+				a.Z[o] = z;
+				if (EPI == EPI_HIDDEN)
+					a.out[o] = gelu(z);
+				if (EPI == EPI_LOSS) {
+					const float d = z - a.T[(size_t)(a.tIdx ? a.tIdx[i] : (uint32_t)i) * a.N + j];
+					a.out[o] = a.scale * d;
+					d2 = (double)d * (double)d;
+				}
+			}
 		}
 	}
-}
-
-// dZ = dH * GELU'(Z) in place
-__global__ void gelu_backward_kernel(float* __restrict__ dH, const float* __restrict__ Z, size_t n)
-{
-	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n)
-		dH[i] *= gelu_grad(Z[i]);
-}
-
-// db[n] = sum over rows of dZ[row][n], rows in order
-__global__ void column_sum_kernel(const float* __restrict__ dZ, int rows, int cols, float* __restrict__ db)
-{
-	const int c = blockIdx.x * blockDim.x + threadIdx.x;
-	if (c >= cols)
-		return;
-	float s = 0.f;
-	for (int r = 0; r < rows; ++r)
-		s += dZ[(size_t)r * cols + c];
-	db[c] = s;
-}
-
-// dY = 2 (Y - T) / n and per-row squared errors (summed in order afterwards)
-__global__ void mse_kernel(const float* __restrict__ Y, const float* __restrict__ T, int rows, int cols,
-                           float* __restrict__ dY, float* __restrict__ rowLoss)
-{
-	const int r = blockIdx.x * blockDim.x + threadIdx.x;
-	if (r >= rows)
-		return;
-	const float scale = 2.f / ((float)rows * (float)cols);
-	float s = 0.f;
-	for (int c = 0; c < cols; ++c) {
-		const float d = Y[(size_t)r * cols + c] - T[(size_t)r * cols + c];
-		dY[(size_t)r * cols + c] = scale * d;
-		s += d * d;
+	if (EPI == EPI_LOSS) {
+		if (t < 256)
+			sq[t] = d2;
+		__syncthreads();
+		for (int w = 128; w > 0; w >>= 1) {
+			if (t < w)
+				sq[t] += sq[t + w];
+			__syncthreads();
+		}
+		if (t == 0)
+			a.tileLoss[blockIdx.x] = sq[0];
 	}
-	rowLoss[r] = s;
 }
 
-__global__ void loss_total_kernel(const float* __restrict__ rowLoss, int rows, int cols, float* __restrict__ loss,
-                                  double* __restrict__ epochSum)
-{
-	if (threadIdx.x != 0 || blockIdx.x != 0)
-		return;
-	double s = 0.;
-	for (int r = 0; r < rows; ++r)
-		s += rowLoss[r];
-	const float l = (float)(s / ((double)rows * (double)cols));
-	*loss = l;
-	if (epochSum)
-		*epochSum += l;
-}
+// Weight and bias gradients of all layers, and Adam: layer l's parameters are
+// the (nIn + 1) x nOut matrix whose last row is the bias, and their gradient is
+// [in, 1]^T dZ.  A workgroup owns 16 x 64 parameters: a wave computes 16 x 16
+// gradients, and after an exchange through LDS a thread updates four consecutive
+// parameters.  Bound by the parameters' and both moments' traffic (24 bytes each,
+// read and written: 24 MB at the initializer's size): those loads are in flight
+// during the product, and the gradient itself never goes through memory when
+// training (10.7 us for the million parameters of the initializer's network; the
+// products, column sums and Adam as kernels of their own took 100 us a step).
+constexpr int kMaxLayers = 17;
+constexpr int kDwDeep = 16;  // rows of the batch per lane quarter in flight
 
-__global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m1,
-                            float* __restrict__ m2, size_t n, float lr, float c1, float c2)
-{
-	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	const float gi = g[i];
-	const float a = 0.9f * m1[i] + 0.1f * gi;
-	const float b = 0.999f * m2[i] + 0.001f * gi * gi;
-	m1[i] = a;
-	m2[i] = b;
-	p[i] -= lr * (a * c1) / (sqrtf(b * c2) + 1e-8f);
-}
+struct DwArgs {
+	const float* in[kMaxLayers];   // [rows][nIn] (layer 0: rows through rowIdx)
+	const float* dZ[kMaxLayers];   // [rows][nOut]
+	int nIn[kMaxLayers], nOut[kMaxLayers];
+	uint32_t block0[kMaxLayers + 1];  // first workgroup of each layer
+	uint64_t off[kMaxLayers];         // first parameter of each layer
+	int nLayers, rows;
+	const uint32_t* rowIdx;
+	float *p, *m1, *m2;  // Adam; p null: the gradient goes to g
+	float* g;
+	float lr, c1, c2;
+	const double* tileLoss;  // summed in a fixed order by the first wave
+	uint32_t nTileLoss;
+	double invN;
+	float* loss;
+	double* epochSum;        // loss added if not null
+};
 
-// rows idx[r] of X [n][cols] -> out [r][cols]
-__global__ void gather_kernel(const float* __restrict__ X, const uint32_t* __restrict__ idx, int rows, int cols,
-                              float* __restrict__ out)
+__global__ __launch_bounds__(256) void weight_gradient_kernel(const DwArgs a)
 {
-	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= (size_t)rows * cols)
+	if (blockIdx.x == 0 && threadIdx.x < 64) {
+		double s = 0.;
+		for (uint32_t k = threadIdx.x; k < a.nTileLoss; k += 64)
+			s += a.tileLoss[k];
+		for (int d = 32; d >= 1; d >>= 1)
+			s += __shfl_xor(s, d);
+		if (threadIdx.x == 0) {
+			const float l = (float)(s * a.invN);
+			*a.loss = l;
+			if (a.epochSum)
+				*a.epochSum += l;
+		}
+	}
+	int layer = 0;
+	while (layer + 1 < a.nLayers && blockIdx.x >= a.block0[layer + 1])
+		++layer;
+	const int nIn = a.nIn[layer], nOut = a.nOut[layer];
+	const uint32_t blk = blockIdx.x - a.block0[layer];
+	const uint32_t nx = ((uint32_t)nOut + 63) / 64;
+	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+	const int r = lane & 15, q = lane >> 4;
+	const int m0 = (int)(blk / nx) * 16, n0 = (int)(blk % nx) * 64 + 16 * wave;
+	const int m = m0 + r, mc = min(m, nIn - 1), nc = min(n0 + r, nOut - 1);
+	const float* in = a.in[layer];
+	const float* dZ = a.dZ[layer];
+	const uint32_t* rowIdx = layer == 0 ? a.rowIdx : nullptr;
+	// this thread's parameters: row i, columns c .. c + 3 (left of them inside the row)
+	__shared__ float grad[16][64 + 4];
+	const int i = m0 + (int)threadIdx.x / 16, c = (int)(blk % nx) * 64 + 4 * ((int)threadIdx.x % 16);
+	const int left = i <= nIn ? nOut - c : 0;
+	const size_t o = a.off[layer] + (size_t)i * nOut + c;
+	f32x4 p, m1, m2;
+	f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+	for (int r0 = 0; r0 < a.rows; r0 += 4 * kDwDeep) {
+		// every lane loads (clamped to the edge, so that no branch sits between the
+		// loads); rows past the batch are zeroed in both operands, parameter rows and
+		// columns past the edge are not stored
+		float av[kDwDeep], bv[kDwDeep];
+		uint32_t src[kDwDeep];
+#pragma unroll
+		for (int d = 0; d < kDwDeep; ++d)
+			src[d] = (uint32_t)min(r0 + 4 * d + q, a.rows - 1);
+#pragma unroll
+		for (int d = 0; d < kDwDeep; ++d)
+			bv[d] = dZ[(size_t)src[d] * nOut + nc];
+		if (rowIdx) {
+#pragma unroll
+			for (int d = 0; d < kDwDeep; ++d)
+				src[d] = rowIdx[src[d]];
+		}
+#pragma unroll
+		for (int d = 0; d < kDwDeep; ++d)
+			av[d] = in[(size_t)src[d] * nIn + mc];
+		// behind the first operands (loads return in order: in front, the row
+		// indices' wait would be theirs too), before the first product
+		if (r0 == 0 && a.p) {
+			p = load4(a.p + o, left);
+			m1 = load4(a.m1 + o, left);
+			m2 = load4(a.m2 + o, left);
+		}
+		__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+		for (int d = 0; d < kDwDeep; ++d) {
+			const bool rowOk = r0 + 4 * d + q < a.rows;
+			const float x = rowOk ? (m == nIn ? 1.f : av[d]) : 0.f, y = rowOk ? bv[d] : 0.f;
+			acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc, 0, 0, 0);
+		}
+	}
+#pragma unroll
+	for (int v = 0; v < 4; ++v)
+		grad[4 * q + v][16 * wave + r] = acc[v];
+	__syncthreads();
+	f32x4 g;
+#pragma unroll
+	for (int v = 0; v < 4; ++v)
+		g[v] = grad[threadIdx.x / 16][4 * (threadIdx.x % 16) + v];
+	if (!a.p) {
+		store4(a.g + o, g, left);
 		return;
-	const size_t r = i / cols, c = i % cols;
-	out[i] = X[(size_t)idx[r] * cols + c];
+	}
+#pragma unroll
+	for (int v = 0; v < 4; ++v) {
+		m1[v] = 0.9f * m1[v] + 0.1f * g[v];
+		m2[v] = 0.999f * m2[v] + 0.001f * g[v] * g[v];
+		p[v] -= a.lr * (m1[v] * a.c1) / (sqrtf(m2[v] * a.c2) + 1e-8f);
+	}
+	store4(a.p + o, p, left);
+	store4(a.m1 + o, m1, left);
+	store4(a.m2 + o, m2, left);
 }
 
 uint64_t mix64(uint64_t x)
@@ -173,14 +341,16 @@ struct rpwa_mlp {
 	// activations of the current capacity (rows)
 	uint32_t capRows = 0;
 	std::vector<float*> d_Z, d_H;  // per layer: pre-activation [rows][out], activation (hidden)
+	std::vector<float*> d_dZ;      // per layer: dLoss / dZ [rows][out]
 	float* d_x = nullptr;
 	float* d_t = nullptr;
-	float* d_dA = nullptr;  // backward buffers [rows][max width]
-	float* d_dB = nullptr;
-	float* d_rowLoss = nullptr;
+	double* d_tileLoss = nullptr;  // per 16 x 16 tile of the output: sum of squared errors
 	float* d_loss = nullptr;
 	double* d_epoch = nullptr;
-	int maxWidth = 0;
+	// training set of the last rpwa_mlp_train call (grown on demand, freed with the network)
+	float *d_setX = nullptr, *d_setT = nullptr;
+	uint32_t* d_idx = nullptr;
+	size_t capX = 0, capT = 0, capIdx = 0;
 
 	~rpwa_mlp() { release(); }
 	void release_acts()
@@ -189,19 +359,26 @@ struct rpwa_mlp {
 			(void)hipFree(p);
 		for (float* p : d_H)
 			(void)hipFree(p);
+		for (float* p : d_dZ)
+			(void)hipFree(p);
 		d_Z.clear();
 		d_H.clear();
-		for (float** p : {&d_x, &d_t, &d_dA, &d_dB, &d_rowLoss})
+		d_dZ.clear();
+		for (float** p : {&d_x, &d_t})
 			if (*p) {
 				(void)hipFree(*p);
 				*p = nullptr;
 			}
+		if (d_tileLoss) {
+			(void)hipFree(d_tileLoss);
+			d_tileLoss = nullptr;
+		}
 		capRows = 0;
 	}
 	void release()
 	{
 		release_acts();
-		for (float** p : {&d_p, &d_g, &d_m1, &d_m2, &d_loss})
+		for (float** p : {&d_p, &d_g, &d_m1, &d_m2, &d_loss, &d_setX, &d_setT})
 			if (*p) {
 				(void)hipFree(*p);
 				*p = nullptr;
@@ -209,6 +386,10 @@ struct rpwa_mlp {
 		if (d_epoch) {
 			(void)hipFree(d_epoch);
 			d_epoch = nullptr;
+		}
+		if (d_idx) {
+			(void)hipFree(d_idx);
+			d_idx = nullptr;
 		}
 		if (stream) {
 			(void)hipStreamDestroy(stream);
@@ -236,91 +417,148 @@ int ensure_rows(rpwa_mlp* m, uint32_t rows)
 	m->release_acts();
 	const int L = m->nLayers();
 	for (int l = 0; l < L; ++l) {
-		float *z = nullptr, *h = nullptr;
+		float *z = nullptr, *h = nullptr, *dz = nullptr;
 		RPWA_HIP_CHECK(hipMalloc(&z, (size_t)rows * m->dims[l + 1] * sizeof(float)));
 		m->d_Z.push_back(z);
 		if (l + 1 < L) {
 			RPWA_HIP_CHECK(hipMalloc(&h, (size_t)rows * m->dims[l + 1] * sizeof(float)));
 		}
 		m->d_H.push_back(h);
+		RPWA_HIP_CHECK(hipMalloc(&dz, (size_t)rows * m->dims[l + 1] * sizeof(float)));
+		m->d_dZ.push_back(dz);
 	}
 	RPWA_HIP_CHECK(hipMalloc(&m->d_x, (size_t)rows * m->dims[0] * sizeof(float)));
 	RPWA_HIP_CHECK(hipMalloc(&m->d_t, (size_t)rows * m->dims[L] * sizeof(float)));
-	RPWA_HIP_CHECK(hipMalloc(&m->d_dA, (size_t)rows * m->maxWidth * sizeof(float)));
-	RPWA_HIP_CHECK(hipMalloc(&m->d_dB, (size_t)rows * m->maxWidth * sizeof(float)));
-	RPWA_HIP_CHECK(hipMalloc(&m->d_rowLoss, (size_t)rows * sizeof(float)));
+	RPWA_HIP_CHECK(hipMalloc(&m->d_tileLoss,
+	                         (size_t)((rows + 15) / 16) * ((m->dims[L] + 15) / 16) * sizeof(double)));
 	m->capRows = rows;
 	return RPWA_OK;
 }
 
-template <bool TA, bool TB, int EPI>
-int gemm(rpwa_mlp* m, const float* A, int lda, const float* B, int ldb, float* C, int ldc, int M, int N, int K,
-         const float* bias = nullptr, float* H = nullptr)
+template <bool TB, int EPI>
+int gemm(rpwa_mlp* m, const GemmArgs& a)
 {
-	const dim3 grid((N + 63) / 64, (M + 63) / 64);
-	hipLaunchKernelGGL((gemm_kernel<TA, TB, EPI>), grid, dim3(256), 0, m->stream, A, lda, B, ldb, C, ldc, M, N, K,
-	                   bias, H);
+	const dim3 grid((uint32_t)((a.N + 15) / 16) * (uint32_t)((a.M + 15) / 16));
+	hipLaunchKernelGGL((gemm_kernel<TB, EPI>), grid, dim3(kGemmThreads), 0, m->stream, a);
 	RPWA_HIP_CHECK(hipGetLastError());
 	return RPWA_OK;
 }
 
-// forward pass of rows in d_x; output in d_Z[L - 1]
-int forward(rpwa_mlp* m, uint32_t rows)
+// the rows of a pass: consecutive rows of x (and t), or the rows idx of them
+struct Rows {
+	const float *x, *t;
+	const uint32_t* idx;
+	uint32_t n;
+};
+
+// forward pass, output in d_Z[L - 1]; withLoss: also the loss tiles and dZ of the output
+int forward(rpwa_mlp* m, const Rows& rows, bool withLoss)
 {
 	const int L = m->nLayers();
-	const float* in = m->d_x;
 	for (int l = 0; l < L; ++l) {
-		const int nin = m->dims[l], nout = m->dims[l + 1];
-		const float* W = m->d_p + m->wOff[l];
-		const float* b = m->d_p + m->bOff[l];
+		GemmArgs a{};
+		a.A = l ? m->d_H[l - 1] : rows.x;
+		a.rowIdx = l ? nullptr : rows.idx;
+		a.B = m->d_p + m->wOff[l];
+		a.bias = m->d_p + m->bOff[l];
+		a.M = (int)rows.n;
+		a.N = a.ldb = m->dims[l + 1];
+		a.K = a.lda = m->dims[l];
+		a.Z = m->d_Z[l];
 		int rc;
-		if (l + 1 < L)
-			rc = gemm<false, false, EPI_BIAS_GELU>(m, in, nin, W, nout, m->d_Z[l], nout, (int)rows, nout, nin, b,
-			                                       m->d_H[l]);
-		else
-			rc = gemm<false, false, EPI_BIAS>(m, in, nin, W, nout, m->d_Z[l], nout, (int)rows, nout, nin, b);
+		if (l + 1 < L) {
+			a.out = m->d_H[l];
+			rc = gemm<false, EPI_HIDDEN>(m, a);
+		} else if (withLoss) {
+			a.out = m->d_dZ[l];
+			a.T = rows.t;
+			a.scale = 2.f / ((float)a.M * (float)a.N);
+			a.tileLoss = m->d_tileLoss;
+			a.tIdx = rows.idx;
+			rc = gemm<false, EPI_LOSS>(m, a);
+		} else {
+			rc = gemm<false, EPI_OUT>(m, a);
+		}
 		if (rc != RPWA_OK)
 			return rc;
-		in = m->d_H[l];
 	}
 	return RPWA_OK;
 }
 
-// loss (into d_loss, and added to *epochSum if given) and gradient into d_g, for rows of d_x / d_t
-int backward(rpwa_mlp* m, uint32_t rows, double* epochSum)
+// Adam of one step
+struct AdamStep {
+	float lr, c1, c2;
+};
+
+// after forward(withLoss): the loss (into d_loss, and added to *epochSum if
+// given), and the gradient into d_g or, with adam, straight into the update
+int backward(rpwa_mlp* m, const Rows& rows, const AdamStep* adam, double* epochSum)
 {
 	const int L = m->nLayers();
-	const int nOut = m->dims[L];
-	float* dZ = m->d_dA;
-	float* dH = m->d_dB;
-	hipLaunchKernelGGL(mse_kernel, dim3((rows + 255) / 256), dim3(256), 0, m->stream, m->d_Z[L - 1], m->d_t,
-	                   (int)rows, nOut, dZ, m->d_rowLoss);
-	RPWA_HIP_CHECK(hipGetLastError());
-	hipLaunchKernelGGL(loss_total_kernel, dim3(1), dim3(64), 0, m->stream, m->d_rowLoss, (int)rows, nOut, m->d_loss,
-	                   epochSum);
-	RPWA_HIP_CHECK(hipGetLastError());
-	for (int l = L - 1; l >= 0; --l) {
-		const int nin = m->dims[l], nout = m->dims[l + 1];
-		const float* in = l == 0 ? m->d_x : m->d_H[l - 1];
-		// dW = in^T dZ  ([nin][nout]), db = column sums of dZ
-		int rc = gemm<true, false, EPI_STORE>(m, in, nin, dZ, nout, m->d_g + m->wOff[l], nout, nin, nout, (int)rows);
+	for (int l = L - 1; l > 0; --l) {
+		// dZ_{l-1} = (dZ_l W_l^T) GELU'(Z_{l-1})
+		GemmArgs a{};
+		a.A = m->d_dZ[l];
+		a.B = m->d_p + m->wOff[l];
+		a.M = (int)rows.n;
+		a.N = m->dims[l];
+		a.K = a.lda = a.ldb = m->dims[l + 1];
+		a.Z = m->d_Z[l - 1];
+		a.out = m->d_dZ[l - 1];
+		const int rc = gemm<true, EPI_DZ>(m, a);
 		if (rc != RPWA_OK)
 			return rc;
-		hipLaunchKernelGGL(column_sum_kernel, dim3((nout + 255) / 256), dim3(256), 0, m->stream, dZ, (int)rows, nout,
-		                   m->d_g + m->bOff[l]);
-		RPWA_HIP_CHECK(hipGetLastError());
-		if (l > 0) {
-			// dH = dZ W^T ([rows][nin]), then dZ_{l-1} = dH * GELU'(Z_{l-1})
-			rc = gemm<false, true, EPI_STORE>(m, dZ, nout, m->d_p + m->wOff[l], nout, dH, nin, (int)rows, nin, nout);
-			if (rc != RPWA_OK)
-				return rc;
-			const size_t n = (size_t)rows * nin;
-			hipLaunchKernelGGL(gelu_backward_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, m->stream, dH,
-			                   m->d_Z[l - 1], n);
-			RPWA_HIP_CHECK(hipGetLastError());
-			std::swap(dZ, dH);
-		}
 	}
+	DwArgs d{};
+	uint32_t blocks = 0;
+	for (int l = 0; l < L; ++l) {
+		d.in[l] = l ? m->d_H[l - 1] : rows.x;
+		d.dZ[l] = m->d_dZ[l];
+		d.nIn[l] = m->dims[l];
+		d.nOut[l] = m->dims[l + 1];
+		d.off[l] = m->wOff[l];
+		d.block0[l] = blocks;
+		blocks += (uint32_t)((m->dims[l] + 1 + 15) / 16) * (uint32_t)((m->dims[l + 1] + 63) / 64);
+	}
+	d.block0[L] = blocks;
+	d.nLayers = L;
+	d.rows = (int)rows.n;
+	d.rowIdx = rows.idx;
+	if (adam) {
+		d.p = m->d_p;
+		d.m1 = m->d_m1;
+		d.m2 = m->d_m2;
+		d.lr = adam->lr;
+		d.c1 = adam->c1;
+		d.c2 = adam->c2;
+	}
+	d.g = m->d_g;
+	d.tileLoss = m->d_tileLoss;
+	d.nTileLoss = ((rows.n + 15) / 16) * (uint32_t)((m->dims[L] + 15) / 16);
+	d.invN = 1. / ((double)rows.n * (double)m->dims[L]);
+	d.loss = m->d_loss;
+	d.epochSum = epochSum;
+	hipLaunchKernelGGL(weight_gradient_kernel, dim3(blocks), dim3(256), 0, m->stream, d);
+	RPWA_HIP_CHECK(hipGetLastError());
+	return RPWA_OK;
+}
+
+// a device buffer of at least n elements
+template <typename T>
+int grow(T** p, size_t* cap, size_t n)
+{
+	if (n <= *cap)
+		return RPWA_OK;
+	if (*p)
+		(void)hipFree(*p);
+	*p = nullptr;
+	*cap = 0;
+	if (hipMalloc(p, n * sizeof(T)) != hipSuccess) {
+		*p = nullptr;
+		set_error("rpwa_mlp_train: device allocation failed");
+		return RPWA_ERR_NOMEM;
+	}
+	*cap = n;
 	return RPWA_OK;
 }
 
@@ -346,7 +584,6 @@ extern "C" int rpwa_mlp_create(rpwa_mlp** out, int device, uint32_t nIn, uint32_
 	for (uint32_t l = 0; l < nHiddenLayers; ++l)
 		m->dims.push_back((int)nHidden);
 	m->dims.push_back((int)nOut);
-	m->maxWidth = *std::max_element(m->dims.begin(), m->dims.end());
 	std::vector<float> p;
 	for (int l = 0; l < m->nLayers(); ++l) {
 		const int nin = m->dims[l], nout = m->dims[l + 1];
@@ -441,7 +678,7 @@ extern "C" int rpwa_mlp_forward(rpwa_mlp* m, const float* x, uint32_t nRows, flo
 		return rc;
 	RPWA_HIP_CHECK(hipMemcpyAsync(m->d_x, x, (size_t)nRows * m->dims[0] * sizeof(float), hipMemcpyHostToDevice,
 	                              m->stream));
-	if (forward(m, nRows) != RPWA_OK)
+	if (forward(m, Rows{m->d_x, nullptr, nullptr, nRows}, false) != RPWA_OK)
 		return RPWA_ERR_HIP;
 	RPWA_HIP_CHECK(hipMemcpyAsync(y, m->d_Z.back(), (size_t)nRows * m->dims.back() * sizeof(float),
 	                              hipMemcpyDeviceToHost, m->stream));
@@ -465,7 +702,8 @@ extern "C" int rpwa_mlp_loss_grad(rpwa_mlp* m, const float* x, const float* targ
 	                              m->stream));
 	RPWA_HIP_CHECK(hipMemcpyAsync(m->d_t, target, (size_t)nRows * m->dims.back() * sizeof(float),
 	                              hipMemcpyHostToDevice, m->stream));
-	if ((rc = forward(m, nRows)) != RPWA_OK || (rc = backward(m, nRows, nullptr)) != RPWA_OK)
+	const Rows rows{m->d_x, m->d_t, nullptr, nRows};
+	if ((rc = forward(m, rows, true)) != RPWA_OK || (rc = backward(m, rows, nullptr, nullptr)) != RPWA_OK)
 		return rc;
 	RPWA_HIP_CHECK(hipMemcpyAsync(loss, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
 	if (grad)
@@ -488,26 +726,15 @@ extern "C" int rpwa_mlp_train(rpwa_mlp* m, const float* x, const float* target, 
 	if (rc != RPWA_OK)
 		return rc;
 	const int nIn = m->dims[0], nOut = m->dims.back();
-	float *d_X = nullptr, *d_T = nullptr;
-	uint32_t* d_idx = nullptr;
-	auto cleanup = [&]() {
-		if (d_X)
-			(void)hipFree(d_X);
-		if (d_T)
-			(void)hipFree(d_T);
-		if (d_idx)
-			(void)hipFree(d_idx);
-	};
-	if (hipMalloc(&d_X, (size_t)nRows * nIn * sizeof(float)) != hipSuccess ||
-	    hipMalloc(&d_T, (size_t)nRows * nOut * sizeof(float)) != hipSuccess ||
-	    hipMalloc(&d_idx, (size_t)nRows * sizeof(uint32_t)) != hipSuccess) {
-		cleanup();
-		set_error("rpwa_mlp_train: device allocation failed");
-		return RPWA_ERR_NOMEM;
-	}
-	if (hipMemcpy(d_X, x, (size_t)nRows * nIn * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
-	    hipMemcpy(d_T, target, (size_t)nRows * nOut * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
-		cleanup();
+	if ((rc = grow(&m->d_setX, &m->capX, (size_t)nRows * nIn)) != RPWA_OK ||
+	    (rc = grow(&m->d_setT, &m->capT, (size_t)nRows * nOut)) != RPWA_OK ||
+	    (rc = grow(&m->d_idx, &m->capIdx, (size_t)nRows)) != RPWA_OK)
+		return rc;
+	if (hipMemcpyAsync(m->d_setX, x, (size_t)nRows * nIn * sizeof(float), hipMemcpyHostToDevice, m->stream) !=
+	        hipSuccess ||
+	    hipMemcpyAsync(m->d_setT, target, (size_t)nRows * nOut * sizeof(float), hipMemcpyHostToDevice, m->stream) !=
+	        hipSuccess ||
+	    hipStreamSynchronize(m->stream) != hipSuccess) {
 		set_error("rpwa_mlp_train: copy failed");
 		return RPWA_ERR_HIP;
 	}
@@ -520,7 +747,7 @@ extern "C" int rpwa_mlp_train(rpwa_mlp* m, const float* x, const float* target, 
 			const uint64_t h = mix64(seed ^ mix64(((uint64_t)epoch << 32) + i));
 			std::swap(perm[i], perm[(uint32_t)(h % (i + 1))]);
 		}
-		if (hipMemcpyAsync(d_idx, perm.data(), nRows * sizeof(uint32_t), hipMemcpyHostToDevice, m->stream) !=
+		if (hipMemcpyAsync(m->d_idx, perm.data(), nRows * sizeof(uint32_t), hipMemcpyHostToDevice, m->stream) !=
 		        hipSuccess ||
 		    hipMemsetAsync(m->d_epoch, 0, sizeof(double), m->stream) != hipSuccess) {
 			rc = RPWA_ERR_HIP;
@@ -528,20 +755,12 @@ extern "C" int rpwa_mlp_train(rpwa_mlp* m, const float* x, const float* target, 
 		}
 		const uint32_t nBatches = nRows / B;  // full batches only
 		for (uint32_t bi = 0; bi < nBatches && rc == RPWA_OK; ++bi) {
-			const size_t ni = (size_t)B * nIn, no = (size_t)B * nOut;
-			hipLaunchKernelGGL(gather_kernel, dim3((uint32_t)((ni + 255) / 256)), dim3(256), 0, m->stream, d_X,
-			                   d_idx + (size_t)bi * B, (int)B, nIn, m->d_x);
-			hipLaunchKernelGGL(gather_kernel, dim3((uint32_t)((no + 255) / 256)), dim3(256), 0, m->stream, d_T,
-			                   d_idx + (size_t)bi * B, (int)B, nOut, m->d_t);
-			if ((rc = forward(m, B)) != RPWA_OK || (rc = backward(m, B, m->d_epoch)) != RPWA_OK)
-				break;
 			++m->adamStep;
-			const float c1 = (float)(1. / (1. - std::pow(0.9, (double)m->adamStep)));
-			const float c2 = (float)(1. / (1. - std::pow(0.999, (double)m->adamStep)));
-			hipLaunchKernelGGL(adam_kernel, dim3((uint32_t)((m->nParams + 255) / 256)), dim3(256), 0, m->stream,
-			                   m->d_p, m->d_g, m->d_m1, m->d_m2, m->nParams, lr, c1, c2);
-			if (hipGetLastError() != hipSuccess)
-				rc = RPWA_ERR_HIP;
+			const AdamStep adam{lr, (float)(1. / (1. - std::pow(0.9, (double)m->adamStep))),
+			                    (float)(1. / (1. - std::pow(0.999, (double)m->adamStep)))};
+			const Rows rows{m->d_setX, m->d_setT, m->d_idx + (size_t)bi * B, B};
+			if ((rc = forward(m, rows, true)) == RPWA_OK)
+				rc = backward(m, rows, &adam, m->d_epoch);
 		}
 		if (rc == RPWA_OK && lossPerEpoch) {
 			double s = 0.;
@@ -553,7 +772,6 @@ extern "C" int rpwa_mlp_train(rpwa_mlp* m, const float* x, const float* target, 
 	}
 	if (hipStreamSynchronize(m->stream) != hipSuccess && rc == RPWA_OK)
 		rc = RPWA_ERR_HIP;
-	cleanup();
 	if (rc != RPWA_OK && rpwa_last_error()[0] == 0)
 		set_error("rpwa_mlp_train: a kernel launch or copy failed");
 	return rc;

@@ -1,0 +1,46 @@
+"""The network's kernels at the edges of their tiles (16 x 16 outputs, 16-deep
+groups of K, 16 x 64 parameters, 64 batch rows per step) against the FP64 oracle.
+
+Tolerances as in test_gpu_initializer.py (FP32 sums of at most a few hundred
+terms, relative to the largest magnitude: forward 1e-5, gradient 1e-4).  The
+first Adam step moves a parameter by lr g / (|g| + 1e-8): exact to the rounding
+of the parameter (2^-24 relative, and of the quotient, 4 of them) wherever the
+gradient's sign is beyond its own error."""
+import numpy as np
+import pytest
+
+from oracle import mlp_oracle as M
+
+pytestmark = pytest.mark.gpu
+
+# (nIn, nHidden, nHiddenLayers, nOut), rows
+EDGES = [((1, 1, 1, 1), 1), ((3, 5, 0, 2), 4), ((15, 16, 1, 17), 16), ((16, 17, 2, 15), 17), ((17, 64, 1, 65), 63),
+         ((31, 33, 16, 3), 64), ((512, 15, 1, 1), 65), ((129, 48, 2, 63), 130), ((775, 64, 1, 176), 64)]
+
+
+@pytest.mark.parametrize("shape,rows", EDGES)
+def test_edges(gpu, shape, rows):
+    from rootpwa_amd.mlp import MLP
+    rng = np.random.default_rng(rows)
+    net = MLP(*shape, seed=2)
+    p = (rng.normal(size=net.nParams()) / np.sqrt(max(shape[0], shape[1]))).astype(np.float32)
+    x = rng.normal(size=(rows, shape[0])).astype(np.float32)
+    t = rng.normal(size=(rows, shape[3])).astype(np.float32)
+    net.setParams(p)
+    layers = M.unpack(p.astype(np.float64), *shape)
+    y, _ = M.forward(layers, x)
+    assert np.max(np.abs(net.forward(x) - y)) <= 1e-5 * np.max(np.abs(y))
+    loss, g = net.lossGrad(x, t)
+    lref, gref = M.loss_grad(layers, x, t)
+    assert abs(loss - lref) <= 1e-5 * lref
+    assert np.max(np.abs(g - gref)) <= 1e-4 * np.max(np.abs(gref))
+    # one batch holding all rows, one step
+    lr = 0.01
+    net.train(x, t, batchSize=rows, epochs=1, lr=lr, seed=1)
+    q = net.params().astype(np.float64)
+    big = np.abs(gref) > 1e-3 * np.max(np.abs(gref))
+    want = p - lr * gref / (np.abs(gref) + 1e-8)
+    err = np.abs(q - want)[big]
+    # relative: 1e-8 / |g| changes by at most the gradient's 10 % error there
+    tol = (2.0 ** -24 * (np.abs(want) + 4 * lr) + lr * 0.1 * 1e-8 / np.abs(gref))[big]
+    assert np.all(err <= tol)

@@ -2,7 +2,7 @@
 //
 // One evaluation of all fits is four kernels, captured once in a hipGraph and
 // replayed for every L-BFGS iteration:
-//   batch_event_kernel   persistent waves; each wave takes work units (bin,
+//   batch_event_kernel   persistent workgroups; each takes work units (bin,
 //                        chunk of 32 tiles of 32 events, group of 16 starts)
 //                        and computes, tile by tile, S = A T (FP32 MFMA),
 //                        sigma, ln sigma (FP64) and G += A^H (S / sigma) (FP32
@@ -16,7 +16,7 @@
 //                        columns, and the list of work units of the next pass
 //                        (only column groups holding a running start).
 // A partial depends only on its chunk and on the start's data, never on the
-// wave that computed it or on which column the start occupies, and the chunk
+// workgroup that computed it or on which column the start occupies, and the chunk
 // partials are summed in chunk order: results do not depend on timing, on the
 // grid, or on how many other fits are still running.
 #include <hip/hip_runtime.h>
@@ -40,25 +40,41 @@ namespace rpwa_amd {
 namespace {
 
 constexpr int kCols = 64;        // starts per bin: 4 column groups
-constexpr int kGroup = 16;       // starts per column group (one wave: 32 MFMA columns)
-constexpr int kEv = 32;          // events per tile (MFMA 32x32 rows)
+constexpr int kGroup = 16;       // starts per column group (32 MFMA columns: Re, Im)
+constexpr int kEv = 32;          // events per tile
 constexpr int kChunkTiles = 32;  // tiles per work unit (1024 events): short units keep a batched fit's tail short
-constexpr int kThreads = 256;    // 4 independent waves per block
+constexpr int kThreads = 256;    // 4 waves, one work unit
+constexpr int kHalf = 8;         // starts per half group: 16 columns, one product's width
+constexpr uint32_t kFull = 8;    // unit code chunk * 16 + first half group, + kFull for up to four of them
 constexpr int kMaxMem = 16;      // L-BFGS correction pairs
-constexpr int kTStride = kGroup + 1;  // LDS row of one wave's production amplitudes (float2)
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-// global-address-space views, so amplitude loads are global (not flat) loads
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(1))) const f32x4 gfloat4;
-typedef __attribute__((address_space(1))) const float gfloat;
+
+// Amplitude storage: per tile of 32 events [event][2 Wp] floats, the LDS image
+// that the event kernel reads, so that a tile is one contiguous copy.  Wave
+// components (2 i, 2 i + 1 = Re, Im of wave i) are permuted within each block of
+// 16 such that lane quarter q of a 16x16x4 product finds its components of four
+// consecutive steps in one 16-byte unit: position 4 q + i holds component
+// comp_of(q, i).  The steps thus take the components in the order 0 4 1 5 | 2 6
+// 3 7 | 8 12 9 13 | 10 14 11 15.  The units of a row are exchanged (XOR, within
+// blocks of 4 or 16) by the row, so that reading one unit of many rows uses all
+// banks.  ks = 2 Wp / 16.
+__host__ __device__ constexpr uint32_t tile_bytes(uint32_t ks) { return 2048u * ks; }
+__host__ __device__ constexpr uint32_t comp_of(uint32_t q, uint32_t i)
+{
+	return 4 * (q & 1) + (q >> 1) + 2 * (i & 1) + 8 * (i >> 1);
+}
+__host__ __device__ constexpr uint32_t swizzle(uint32_t ks, uint32_t row)
+{
+	return (ks & 3) == 0 ? row & 15 : (ks & 1) ? (row >> 2) & 3 : (row >> 1) & 3;
+}
 
 struct BatchEventArgs {
-	const float* const* binAmps;  // per bin: [tiles * 32][rowLen] float (complex64 pairs)
+	const char* const* binAmps;   // per bin: [tiles][32][rowLen] floats, permuted
 	const uint32_t* chunkBin;     // [nChunks]
 	const uint32_t* chunkTile0;   // [nChunks] first tile of the chunk within its bin
 	const uint32_t* nEvents;      // [nBins]
-	const uint32_t* units;        // [nChunks * 4] chunk * 4 + column group, this pass
+	const uint32_t* units;        // [nChunks * 4] work units of this pass (unit code)
 	const uint32_t* nUnits;       // [1]
 	const int32_t* colMap;        // [nBins][64] start held by each column (-1: none)
 	const float* T32;             // [nBins][64][rowLen] by start
@@ -82,201 +98,448 @@ __device__ __forceinline__ double swap_pair_d(double v)
 	return __longlong_as_double((long long)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
 }
 
-// One wave per work unit.  Lane (h, j): MFMA column j = (start slot j / 2 of
-// the group, Re / Im of S by j % 2); MFMA rows are events (S = A T) or wave
-// components (G = A^T V).  KQ = Wp / 4.
-template <int KQ>
-__global__ __launch_bounds__(kThreads, 2) void batch_event_kernel(const BatchEventArgs a)
+// 16 bytes per lane of global memory straight into LDS: lane l of the wave
+// writes base + 16 l.  In assembly because the compiler would let every later
+// LDS read wait for it; there is no register result, and the waits are explicit
+// (dma_wait before the barrier that publishes the data).
+__device__ __forceinline__ void dma16(const char* src, uint32_t base)
 {
-	constexpr int NT = (KQ + 3) / 4;            // tiles of 32 wave components
-	constexpr uint32_t rowLen = 8 * KQ;         // 2 Wp floats per event
-	constexpr uint32_t Wp = 4 * KQ;
-	constexpr int lastCols = (int)rowLen - 32 * (NT - 1);  // valid columns of the last component tile
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(base), "v"(src) : "memory", "m0");
+}
+__device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-	__shared__ float2 Tlds[kThreads / 64][Wp * kTStride];
-	const int lane = threadIdx.x & 63;
+// LDS of one workgroup: two tile buffers, V and sigma of a tile.  At 88 waves
+// 53.4 KB, so that three workgroups fit on a CU.
+constexpr uint32_t kVStride = 33;  // floats per event of V
+constexpr uint32_t event_lds(uint32_t ks)
+{
+	return 2 * tile_bytes(ks) + kEv * kVStride * (uint32_t)sizeof(float) + kEv * kGroup * (uint32_t)sizeof(double);
+}
+
+// Products on v_mfma_f32_16x16x4_f32.  It and the other FP32 shapes add their
+// products one after the other, each rounded as an fma, so neither the shape nor
+// the wave changes a sum, only the order of its terms does: components as in
+// comp_of for S, events 0 4 1 5 | 2 6 3 7 | 8 12 ... of every tile for G.
+//
+// sigma = |S|^2 + flat^2 in FP64 from the Re / Im pair of lanes, 1 / sigma of the
+// hardware reciprocal, and the running product of sigma as m 2^e with m in
+// [1, 2), renormalised per tile.
+struct LogProduct {
+	double mant = 1., invSum = 0.;
+	int expo = 0;
+	__device__ __forceinline__ void add(double sig, double inv)
+	{
+		mant *= sig;
+		invSum += inv;
+	}
+	__device__ __forceinline__ void renormalise()  // sigma > 0 is finite or inf / nan
+	{
+		const uint64_t ub = (uint64_t)__double_as_longlong(mant);
+		const int e = (int)((ub >> 52) & 0x7FF);
+		if (e != 0 && e != 0x7FF) {
+			expo += e - 1023;
+			mant = __longlong_as_double((long long)((ub & 0x800FFFFFFFFFFFFFull) | (1023ull << 52)));
+		}
+	}
+	__device__ __forceinline__ double ln() const { return log(mant) + (double)expo * 0.69314718055994530942; }
+};
+
+// what both kinds of unit share: the chunk, its amplitudes and the lane's place
+template <int KS>
+struct UnitBase {
+	static constexpr uint32_t rowLen = 16 * KS;  // 2 Wp floats per event
+	static constexpr uint32_t kRowB = 4 * rowLen;
+	static constexpr uint32_t kTile = tile_bytes(KS);
+	static constexpr int kDma = 2 * KS;          // 1 KB copies per tile
+	const BatchEventArgs& a;
+	char* smem;
+	uint32_t lds0;
+	int lane, wave, r, q, cout;
+	uint32_t cg, b, nEv, tile0, tile1;
+	const char* amps;
+
+	__device__ UnitBase(const BatchEventArgs& args, char* sm, uint32_t chunk) : a(args), smem(sm)
+	{
+		lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+		lane = threadIdx.x & 63;
+		wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+		r = lane & 15, q = lane >> 4;
+		cout = r & 1;  // this lane's column: Re (0) or Im (1) of S
+		cg = chunk;
+		b = a.chunkBin[cg];
+		nEv = a.nEvents[b];
+		tile0 = a.chunkTile0[cg];
+		tile1 = min(tile0 + (uint32_t)kChunkTiles, (nEv + kEv - 1) / kEv);
+		amps = a.binAmps[b];
+	}
+	__device__ __forceinline__ void copy_tile(uint32_t t, uint32_t buf) const
+	{
+		for (int c = wave; c < kDma; c += 4)
+			dma16(amps + (size_t)t * kTile + 1024 * c + 16 * lane, lds0 + buf + 1024 * c);
+	}
+	// T of column r of half group `half` as the B operand: [Sre Sim] = [Are Aim]
+	// [[Tre Tim] [-Tim Tre]]; the quarters 0, 1 hold the real components, 2, 3 the
+	// imaginary.  Returns flat^2 (1 for a column without a start)
+	__device__ __forceinline__ double load_t(uint32_t half, float (&T)[4 * KS]) const
+	{
+		const int start = a.colMap[b * kCols + kHalf * half + (r >> 1)];
+		const float2* Tb = reinterpret_cast<const float2*>(a.T32 + ((size_t)b * kCols + max(start, 0)) * rowLen);
+#pragma unroll
+		for (int s = 0; s < KS; ++s)
+#pragma unroll
+			for (int i = 0; i < 4; ++i) {
+				const float2 t = Tb[8 * s + 2 * (q & 1) + (i & 1) + 4 * (i >> 1)];
+				const float v = q < 2 ? (cout ? t.y : t.x) : (cout ? t.x : -t.y);
+				T[4 * s + i] = start >= 0 ? v : 0.f;
+			}
+		return start >= 0 ? a.flat2[(size_t)b * kCols + start] : 1.;
+	}
+	// partial sums of component block blk: register v is position 4 q + v, component
+	// comp_of(q, v), so the real and the imaginary component of a wave are in lanes
+	// 32 apart, columns 2 s, 2 s + 1 in neighbouring lanes: Re G = Xre[2s] +
+	// Xim[2s+1], Im G = Xre[2s+1] - Xim[2s]
+	__device__ __forceinline__ void put(uint32_t half, int blk, const f32x4 X) const
+	{
+		float* pg = a.partG + (size_t)(4 * cg + (half >> 1)) * (rowLen * kGroup) +
+		            ((half & 1) * kHalf + (r >> 1)) * rowLen + 16 * blk;
+#pragma unroll
+		for (int v = 0; v < 4; ++v) {
+			const float pair = swap_pair(X[v]);          // the other column's
+			const float far0 = __shfl_xor(X[v], 32);     // the other component's
+			const float far1 = __shfl_xor(pair, 32);
+			if (q < 2 && cout == 0) {
+				pg[comp_of(q, v)] = X[v] + far1;
+				pg[comp_of(q, v) + 1] = pair - far0;
+			}
+		}
+	}
+	__device__ __forceinline__ void put_sums(uint32_t half, uint32_t slot, double ln, double inv) const
+	{
+		const size_t o = (size_t)(4 * cg + (half >> 1)) * kGroup + (half & 1) * kHalf + slot;
+		a.partLn[o] = ln;
+		a.partInv[o] = inv;
+	}
+};
+
+// A unit of up to four half groups (three or four; a batch's first iterations):
+// wave w takes half group first + w, whole: S of the tile's 32 events in two
+// products, V = S / sigma as it stands as the other operand of G (row m = 4 q + v
+// of S's product mb is the event of step 4 mb + v of G's in quarter q), G of all
+// components.  The waves share only the tile: one barrier per tile.  Bound by
+// FP32 MFMA: 16 KS instructions of 32 cycles per wave and tile.
+template <int KS>
+__device__ __forceinline__ void full_unit(const BatchEventArgs& a, char* smem, uint32_t chunk, uint32_t first)
+{
+	typedef UnitBase<KS> U;
+	const U u(a, smem, chunk);
+	const int r = u.r, q = u.q;
+	const uint32_t half = first + u.wave;
+	const bool active = half < kCols / kHalf && a.colMap[u.b * kCols + kHalf * (half & 7)] >= 0;
+	__syncthreads();  // the previous unit is done with LDS
+	u.copy_tile(u.tile0, 0);
+	// S operand of product mb: row r = 4 qr + vr is event 8 ((4 mb + vr) / 2) + 2 (vr % 2) + 4 (qr % 2) + qr / 2
+	uint32_t sOff[2][4];
+#pragma unroll
+	for (uint32_t mb = 0; mb < 2; ++mb) {
+		const uint32_t st = 4 * mb + (r & 3), qr = r >> 2;
+		const uint32_t ev = 8 * (st >> 1) + 2 * (st & 1) + 4 * (qr & 1) + (qr >> 1);
+#pragma unroll
+		for (uint32_t s = 0; s < 4; ++s)
+			sOff[mb][s] = ev * U::kRowB + 16 * ((4 * s + q) ^ swizzle(KS, ev));
+	}
+	// G operand: position r of block x, in step st the row (event) ev0 + gEv0 with
+	// ev0 = 8 (st / 2) + 2 (st % 2): byte gOff[gBase(st)] + ev0 kRowB + 64 gBlock(x, st),
+	// rows of a multiple of 16 units with the base chosen by x too
+	// (the step's and the quarter's parts of the row's swizzle do not share bits)
+	const uint32_t gEv0 = 4 * (q & 1) + (q >> 1);
+	uint32_t gOff[2][2];
+#pragma unroll
+	for (uint32_t k = 0; k < 2; ++k)
+#pragma unroll
+		for (uint32_t odd = 0; odd < 2; ++odd)
+			gOff[k][odd] = gEv0 * U::kRowB + 4 * (r & 3) +
+			               16 * ((4 * odd + (r >> 2)) ^ swizzle(KS, gEv0 + ((KS & 1) ? 8 : 2) * k));
+	auto gByte = [&](int x, int st) {
+		const int k = (KS & 1) ? (st >> 1) & 1 : st & 1;
+		const int pairBlk = (KS & 3) == 0 ? (x >> 1) ^ ((st >> 1) & 1) : x >> 1;
+		return gOff[k][x & 1] + 128 * pairBlk + (8 * (st >> 1) + 2 * (st & 1)) * U::kRowB;
+	};
+	float T[4 * KS];
+	const double f2 = u.load_t(half & 7, T);
+	f32x4 G[KS];
+#pragma unroll
+	for (int x = 0; x < KS; ++x)
+		G[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+	LogProduct lp;
+
+	for (uint32_t t = u.tile0; t < u.tile1; ++t) {
+		const uint32_t buf = ((t - u.tile0) & 1) * U::kTile;
+		dma_wait();
+		__syncthreads();  // the tile is in LDS, and the other buffer is free
+		if (t + 1 < u.tile1)
+			u.copy_tile(t + 1, U::kTile - buf);
+		if (!active)
+			continue;
+		const char* const tile = smem + buf;
+		// ---- S (operands read two units ahead; the scheduling barriers keep the
+		// compiler from reading all of them at once) ----
+		f32x4 S[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+		constexpr int kAhead = KS < 3 ? KS : 3;
+		f32x4 sv[kAhead][2];
+		auto sRead = [&](int s) {
+#pragma unroll
+			for (int mb = 0; mb < 2; ++mb)
+				sv[s % kAhead][mb] = *reinterpret_cast<const f32x4*>(tile + sOff[mb][s & 3] + 256 * (s >> 2));
+		};
+#pragma unroll
+		for (int s = 0; s < kAhead - 1; ++s)
+			sRead(s);
+#pragma unroll
+		for (int s = 0; s < KS; ++s) {
+			if (s + kAhead - 1 < KS)
+				sRead(s + kAhead - 1);
+#pragma unroll
+			for (int i = 0; i < 4; ++i)
+#pragma unroll
+				for (int mb = 0; mb < 2; ++mb)
+					S[mb] = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[s % kAhead][mb][i], T[4 * s + i], S[mb], 0, 0, 0);
+			__builtin_amdgcn_sched_barrier(0);
+		}
+		// ---- V ----
+		const uint32_t evBase = t * kEv + gEv0;
+		const bool whole = (t + 1) * kEv <= u.nEv;
+		float V[8];
+#pragma unroll
+		for (int st = 0; st < 8; ++st) {
+			const float own = S[st >> 2][st & 3];
+			const float other = swap_pair(own);
+			const float re = u.cout ? other : own, im = u.cout ? own : other;
+			double sig = fma((double)re, (double)re, fma((double)im, (double)im, f2));
+			const bool valid = whole || evBase + 8 * (st >> 1) + 2 * (st & 1) < u.nEv;
+			sig = valid ? sig : 1.;
+			const float inv = __builtin_amdgcn_rcpf((float)sig);
+			V[st] = valid ? own * inv : 0.f;
+			lp.add(sig, valid ? (double)inv : 0.);
+		}
+		lp.renormalise();
+		// ---- G (operands read a step ahead) ----
+		float gv[2][KS];
+		auto gRead = [&](int st) {
+#pragma unroll
+			for (int x = 0; x < KS; ++x)
+				gv[st & 1][x] = *reinterpret_cast<const float*>(tile + gByte(x, st));
+		};
+		gRead(0);
+#pragma unroll
+		for (int st = 0; st < 8; ++st) {
+			if (st < 7)
+				gRead(st + 1);
+#pragma unroll
+			for (int x = 0; x < KS; ++x)
+				G[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(gv[st & 1][x], V[st], G[x], 0, 0, 0);
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	}
+	if (!active)
+		return;
+#pragma unroll
+	for (int x = 0; x < KS; ++x)
+		u.put(half, x, G[x]);
+	// quarter q holds the events of bit 2 = q % 2 and bit 0 = q / 2
+	double lnv = lp.ln(), inv = lp.invSum;
+	lnv += __shfl_xor(lnv, 32);
+	inv += __shfl_xor(inv, 32);
+	lnv += __shfl_xor(lnv, 16);
+	inv += __shfl_xor(inv, 16);
+	if (q == 0 && u.cout == 0)
+		u.put_sums(half, r >> 1, lnv, inv);
+}
+
+// A unit of one or two half groups (few starts, or the tail of a batched fit,
+// where the time of an iteration is that of one unit): the four waves share it.
+//   S: wave w computes events 16 (w / 2) .. + 15 of half group first + w % 2; V and
+//      sigma go to LDS;
+//   G: wave w keeps the component blocks w / 2, w / 2 + 2, ... of that half group,
+//      each event's V from LDS; wave 2 also multiplies up sigma.
+// Two barriers per tile (the tile is in LDS; V is).  A wave's latency over 32 tiles with the
+// operands straight from L1 was 250 us of every iteration.
+template <int KS>
+__device__ __forceinline__ void shared_unit(const BatchEventArgs& a, char* smem, uint32_t chunk, uint32_t first)
+{
+	typedef UnitBase<KS> U;
+	constexpr int NB = (KS + 1) / 2;            // component blocks of a wave (waves 2, 3 may have one fewer)
+	const U u(a, smem, chunk);
+	const int r = u.r, q = u.q, cout = u.cout, lane = u.lane;
+	float* const vL = reinterpret_cast<float*>(smem + 2 * U::kTile);
+	double* const sigL = reinterpret_cast<double*>(smem + 2 * U::kTile + kEv * kVStride * sizeof(float));
+	const uint32_t wh = u.wave >> 1;
+	const uint32_t half = first + (u.wave & 1);
+	const uint32_t col = 16 * (u.wave & 1) + r;   // column of the two half groups' 32
+	const bool active = a.colMap[u.b * kCols + kHalf * half] >= 0;
+	__syncthreads();  // the previous unit is done with LDS
+	u.copy_tile(u.tile0, 0);
+	// S operand: row (event) 16 wh + r, units 4 s + q: byte sOff[s % 4] + 256 (s / 4)
+	uint32_t sOff[4];
+#pragma unroll
+	for (uint32_t s = 0; s < 4; ++s)
+		sOff[s] = (16 * wh + r) * U::kRowB + 16 * ((4 * s + q) ^ swizzle(KS, 16 * wh + r));
+	// G operand as in full_unit, of the blocks 2 x + wh
+	const uint32_t gEv0 = 4 * (q & 1) + (q >> 1);
+	uint32_t gOff[2];
+#pragma unroll
+	for (uint32_t k = 0; k < 2; ++k)
+		gOff[k] = gEv0 * U::kRowB + 4 * (r & 3) + 16 * ((4 * wh + (r >> 2)) ^ swizzle(KS, gEv0 + ((KS & 1) ? 8 : 2) * k));
+	auto gByte = [&](int x, int st) {
+		const int pairBlk = (KS & 3) == 0 ? x ^ ((st >> 1) & 1) : x;
+		return gOff[(KS & 1) ? (st >> 1) & 1 : st & 1] + 128 * pairBlk + (8 * (st >> 1) + 2 * (st & 1)) * U::kRowB;
+	};
+	float T[4 * KS];
+	const double f2 = u.load_t(half, T);
+	f32x4 G[NB];
+#pragma unroll
+	for (int x = 0; x < NB; ++x)
+		G[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+	// wave 2, lane (h, j): the events of bit 2 = h and bit 0 = j % 2 of start slot j / 2
+	LogProduct lp;
 	const int h = lane >> 5, j = lane & 31;
-	const int cout = j & 1;                     // this lane's column: Re (0) or Im (1) of S
-	float2* Tw = Tlds[threadIdx.x >> 6];
-	const uint32_t nWaves = gridDim.x * (kThreads / 64);
-	const uint32_t nUnits = *a.nUnits;
 
-	for (uint32_t u = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6); u < nUnits; u += nWaves) {
-		const uint32_t unit = a.units[u];
-		const uint32_t cg = unit >> 2, q = unit & 3;
-		const uint32_t b = a.chunkBin[cg];
-		const uint32_t nEv = a.nEvents[b];
-		const uint32_t tile0 = a.chunkTile0[cg];
-		const uint32_t tile1 = min(tile0 + (uint32_t)kChunkTiles, (nEv + kEv - 1) / kEv);
-		const int start = a.colMap[b * kCols + kGroup * q + (j >> 1)];
-
-		// production amplitudes of the group's 16 starts in this wave's LDS
-		// region, [wave i][start slot] (Re, Im); padding columns are zero
-		{
-			const int* cm = a.colMap + b * kCols + kGroup * q;
-			for (int idx = lane; idx < (int)Wp * kGroup; idx += 64) {
-				const int i = idx / kGroup, sl = idx % kGroup;
-				const int st = cm[sl];
-				float2 v = make_float2(0.f, 0.f);
-				if (st >= 0) {
-					const float* Tb = a.T32 + ((size_t)b * kCols + st) * rowLen;
-					v = make_float2(Tb[2 * i], Tb[2 * i + 1]);
-				}
-				Tw[i * kTStride + sl] = v;
-			}
-			__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-			__builtin_amdgcn_wave_barrier();
-			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-		}
-		const double f2 = start >= 0 ? a.flat2[(size_t)b * kCols + start] : 1.;
-		const float2* Tj = Tw + (j >> 1);
-
-		f32x16 X[NT];
+	for (uint32_t t = u.tile0; t < u.tile1; ++t) {
+		const uint32_t buf = ((t - u.tile0) & 1) * U::kTile;
+		dma_wait();
+		__syncthreads();  // the tile is in LDS; the other buffer, V and sigma are free
+		if (t + 1 < u.tile1)
+			u.copy_tile(t + 1, U::kTile - buf);
+		const char* const tile = smem + buf;
+		const uint32_t evBase = t * kEv;
+		const bool whole = evBase + kEv <= u.nEv;
+		if (active) {
+			f32x4 S = f32x4{0.f, 0.f, 0.f, 0.f};
+			constexpr int kAhead = KS < 4 ? KS : 4;
+			f32x4 sv[kAhead];
+			auto sRead = [&](int s) {
+				sv[s % kAhead] = *reinterpret_cast<const f32x4*>(tile + sOff[s & 3] + 256 * (s >> 2));
+			};
 #pragma unroll
-		for (int x = 0; x < NT; ++x)
-			X[x] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-		double mant = 1.;  // running product of sigma, renormalised per tile
-		int expo = 0;
-		double invAcc = 0.;
-		const float* amps = a.binAmps[b];
-
-		// Operands are loaded kPd1 steps (GEMM1) and kPd2 steps (GEMM2) ahead; the
-		// scheduling barriers keep the compiler from hoisting every load of a
-		// tile (register pressure).
-		constexpr int kPd2 = 2;
-		constexpr int kPd1 = KQ < 4 ? KQ : 4;
-		for (uint32_t t = tile0; t < tile1; ++t) {
-			// S[32 events][32 columns] = A_tile T
-			const gfloat4* rowA = (const gfloat4*)(amps + ((size_t)t * kEv + j) * rowLen);
-			f32x16 S = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-			f32x4 avBuf[kPd1];
+			for (int s = 0; s < kAhead - 1; ++s)
+				sRead(s);
 #pragma unroll
-			for (int qq = 0; qq < kPd1; ++qq)
-				avBuf[qq] = rowA[2 * qq + h];
-			float2 t0n = Tj[(2 * h) * kTStride], t1n = Tj[(2 * h + 1) * kTStride];
+			for (int s = 0; s < KS; ++s) {
+				if (s + kAhead - 1 < KS)
+					sRead(s + kAhead - 1);
 #pragma unroll
-			for (int q4 = 0; q4 < KQ; ++q4) {
-				// K steps 4 q4 .. 4 q4 + 3 of lane half h are the wave components
-				// 8 q4 + 4 h + 0..3, i.e. (Re, Im) of waves i0 = 4 q4 + 2 h and i0 + 1;
-				// [Sre Sim] = [Are Aim] [[Tre Tim] [-Tim Tre]]
-				const f32x4 av = avBuf[q4 % kPd1];
-				if (q4 + kPd1 < KQ)
-					avBuf[q4 % kPd1] = rowA[2 * (q4 + kPd1) + h];
-				const float2 t0 = t0n, t1 = t1n;
-				if (q4 + 1 < KQ) {
-					t0n = Tj[(4 * (q4 + 1) + 2 * h) * kTStride];
-					t1n = Tj[(4 * (q4 + 1) + 2 * h + 1) * kTStride];
-				}
-				S = __builtin_amdgcn_mfma_f32_32x32x2f32(av.x, cout ? t0.y : t0.x, S, 0, 0, 0);
-				S = __builtin_amdgcn_mfma_f32_32x32x2f32(av.y, cout ? t0.x : -t0.y, S, 0, 0, 0);
-				S = __builtin_amdgcn_mfma_f32_32x32x2f32(av.z, cout ? t1.y : t1.x, S, 0, 0, 0);
-				S = __builtin_amdgcn_mfma_f32_32x32x2f32(av.w, cout ? t1.x : -t1.y, S, 0, 0, 0);
+				for (int i = 0; i < 4; ++i)
+					S = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[s % kAhead][i], T[4 * s + i], S, 0, 0, 0);
 				__builtin_amdgcn_sched_barrier(0);
 			}
-			// per register p (event 8 (p / 4) + 4 h + p % 4 of the tile, column j):
-			// sigma = |S|^2 + flat^2 (FP64), ln sigma via the running product,
-			// V = S / sigma; then K step p of X[wave components][columns] +=
-			// A_tile^T V, which pairs register p of both lane halves.  Columns of
-			// the last component tile past 2 Wp read within the row's tile and are
-			// zeroed.
-			const uint32_t evBase = t * kEv;
-			const gfloat* tileB = (const gfloat*)(amps + ((size_t)t * kEv + 4 * h) * rowLen);
-			float a2Buf[kPd2][NT];
+			// events 16 wh + 4 q + v: the lanes of a Re / Im pair take the even and the
+			// odd v and exchange 1 / sigma
+			const uint32_t ev0 = 16 * wh + 4 * q;
 #pragma unroll
-			for (int pp = 0; pp < kPd2; ++pp)
-#pragma unroll
-				for (int x = 0; x < NT; ++x)
-					a2Buf[pp][x] = tileB[(8 * (pp >> 2) + (pp & 3)) * rowLen + 32 * x + (x < NT - 1 ? j : min(j, lastCols - 1))];
-#pragma unroll
-			for (int p = 0; p < 16; ++p) {
-				float a2[NT];
-#pragma unroll
-				for (int x = 0; x < NT; ++x)
-					a2[x] = (x < NT - 1 || lastCols >= 32 || j < lastCols) ? a2Buf[p % kPd2][x] : 0.f;
-				if (p + kPd2 < 16) {
-					const int pn = p + kPd2;
-					const gfloat* rowB = tileB + (8 * (pn >> 2) + (pn & 3)) * rowLen;
-#pragma unroll
-					for (int x = 0; x < NT; ++x)
-						a2Buf[p % kPd2][x] = rowB[32 * x + (x < NT - 1 ? j : min(j, lastCols - 1))];
-				}
-				const int row = 8 * (p >> 2) + 4 * h + (p & 3);
-				const bool valid = evBase + (uint32_t)row < nEv;
-				const float me = S[p];
-				const float other = swap_pair(me);
-				const float re = cout ? other : me, im = cout ? me : other;
+			for (int v = 0; v < 4; v += 2) {
+				const float own = cout ? S[v + 1] : S[v];
+				const float other = swap_pair(cout ? S[v] : S[v + 1]);
+				const float re = cout ? other : own, im = cout ? own : other;
 				double sig = fma((double)re, (double)re, fma((double)im, (double)im, f2));
+				const uint32_t ev = ev0 + v + cout;
+				const bool valid = whole || evBase + ev < u.nEv;
 				sig = valid ? sig : 1.;
-				const float inv = __builtin_amdgcn_rcpf((float)sig);
-				const float vp = valid ? me * inv : 0.f;
-				if ((p & 1) == cout) {  // the pair splits the event terms
-					mant *= sig;
-					invAcc += valid ? (double)inv : 0.;
-				}
+				float inv = __builtin_amdgcn_rcpf((float)sig);
+				inv = valid ? inv : 0.f;
+				sigL[ev * kGroup + (col >> 1)] = sig;
+				const float inv2 = swap_pair(inv);
+				vL[(ev0 + v) * kVStride + col] = S[v] * (cout ? inv2 : inv);
+				vL[(ev0 + v + 1) * kVStride + col] = S[v + 1] * (cout ? inv : inv2);
+			}
+		}
+		__syncthreads();  // V and sigma of the tile are in LDS
+		if (active) {
+			float gv[2][NB], vv[2];
+			auto gRead = [&](int st) {
+				vv[st & 1] = vL[(8 * (st >> 1) + 2 * (st & 1) + gEv0) * kVStride + col];
 #pragma unroll
-				for (int x = 0; x < NT; ++x)
-					X[x] = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[x], vp, X[x], 0, 0, 0);
+				for (int x = 0; x < NB; ++x)  // past the last block: some other word, its sums are never used
+					gv[st & 1][x] = *reinterpret_cast<const float*>(tile + gByte(x, st));
+			};
+			gRead(0);
+#pragma unroll
+			for (int st = 0; st < 8; ++st) {
+				if (st < 7)
+					gRead(st + 1);
+#pragma unroll
+				for (int x = 0; x < NB; ++x)
+					if (2 * x + 1 < KS || wh == 0)
+						G[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(gv[st & 1][x], vv[st & 1], G[x], 0, 0, 0);
 				__builtin_amdgcn_sched_barrier(0);
 			}
-			{
-				// mant = m 2^e with m in [1, 2): keep m, carry e (sigma > 0 is finite or inf/nan)
-				const uint64_t ub = (uint64_t)__double_as_longlong(mant);
-				const int e = (int)((ub >> 52) & 0x7FF);
-				if (e != 0 && e != 0x7FF) {
-					expo += e - 1023;
-					mant = __longlong_as_double((long long)((ub & 0x800FFFFFFFFFFFFFull) | (1023ull << 52)));
-				}
-			}
 		}
-
-		// partial of this unit: G_i = sum conj(A_i) V per start slot.  Rows 2i,
-		// 2i+1 of X are registers v, v+1; columns 2s, 2s+1 are lanes j, j^1:
-		// Re G = X[2i][2s] + X[2i+1][2s+1], Im G = X[2i][2s+1] - X[2i+1][2s]
-		const uint32_t slot = cg * 4 + q;
-		float* pg = a.partG + (size_t)slot * Wp * (2 * kGroup);
+		if (u.wave == 2) {
 #pragma unroll
-		for (int x = 0; x < NT; ++x)
-#pragma unroll
-			for (int v = 0; v < 16; v += 2) {
-				const int row0 = 32 * x + 8 * (v >> 2) + 4 * h + (v & 3);
-				const float own0 = X[x][v], own1 = X[x][v + 1];
-				const float p0 = swap_pair(own0), p1 = swap_pair(own1);
-				if (cout == 0 && row0 < (int)rowLen) {
-					const int i = row0 >> 1;
-					pg[((j >> 1) * Wp + i) * 2 + 0] = own0 + p1;
-					pg[((j >> 1) * Wp + i) * 2 + 1] = p0 - own1;
-				}
+			for (int p = 0; p < 8; ++p) {
+				const uint32_t ev = 8 * (p >> 1) + 4 * h + 2 * (p & 1) + (j & 1);
+				const double sig = sigL[ev * kGroup + (j >> 1)];
+				const float inv = __builtin_amdgcn_rcpf((float)sig);
+				lp.add(sig, (whole || evBase + ev < u.nEv) ? (double)inv : 0.);
 			}
-		double lnv = log(mant) + (double)expo * 0.69314718055994530942;
+			lp.renormalise();
+		}
+	}
+	if (active) {
+#pragma unroll
+		for (int x = 0; x < NB; ++x)
+			if (2 * x + (int)wh < KS)
+				u.put(half, 2 * x + wh, G[x]);
+	}
+	if (u.wave == 2) {
+		double lnv = lp.ln(), inv = lp.invSum;
 		lnv += swap_pair_d(lnv);
+		inv += swap_pair_d(inv);
 		lnv += __shfl_xor(lnv, 32);
-		double inv = invAcc + swap_pair_d(invAcc);
 		inv += __shfl_xor(inv, 32);
-		if (h == 0 && cout == 0) {
-			a.partLn[(size_t)slot * kGroup + (j >> 1)] = lnv;
-			a.partInv[(size_t)slot * kGroup + (j >> 1)] = inv;
-		}
+		// an empty second half group has no sums
+		const uint32_t hs = first + (j >> 4);
+		if (h == 0 && (j & 1) == 0 && a.colMap[u.b * kCols + kHalf * hs] >= 0)
+			u.put_sums(hs, (j >> 1) & 7, lnv, inv);
+	}
+}
+
+// One wave per unit with the operands straight from L1 took 5.3 ms for 48 bins of
+// 5.9M events x 88 waves x 64 starts: each amplitude row went through L1 twice
+// per wave, in 32-byte pieces.
+template <int KS>
+__global__ __launch_bounds__(kThreads, KS <= 11 ? 3 : 2) void batch_event_kernel(const BatchEventArgs a)
+{
+	extern __shared__ char smem[];
+	const uint32_t nUnits = *a.nUnits;
+	for (uint32_t k = blockIdx.x; k < nUnits; k += gridDim.x) {
+		// neighbouring units (the two of a chunk) go to one XCD (workgroups of equal
+		// index modulo 8) at about the same time, so that its L2 serves both
+		const uint32_t u = (k | 15u) < nUnits ? (k & ~15u) | ((k & 7) << 1) | ((k >> 3) & 1) : k;
+		const uint32_t unit = a.units[u];
+		if (unit & kFull)
+			full_unit<KS>(a, smem, unit >> 4, unit & 7);
+		else
+			shared_unit<KS>(a, smem, unit >> 4, unit & 7);
 	}
 }
 
 typedef void (*BatchEventKernel)(const BatchEventArgs);
 
-// KQ = Wp / 4, Wp = waves padded to a multiple of 8
-BatchEventKernel pick_event_kernel(int KQ)
+// KS = 2 Wp / 16, Wp = waves padded to a multiple of 8
+BatchEventKernel pick_event_kernel(uint32_t ks)
 {
-	switch (KQ) {
+	switch (ks) {
+	case 1: return batch_event_kernel<1>;
 	case 2: return batch_event_kernel<2>;
+	case 3: return batch_event_kernel<3>;
 	case 4: return batch_event_kernel<4>;
+	case 5: return batch_event_kernel<5>;
 	case 6: return batch_event_kernel<6>;
+	case 7: return batch_event_kernel<7>;
 	case 8: return batch_event_kernel<8>;
+	case 9: return batch_event_kernel<9>;
 	case 10: return batch_event_kernel<10>;
-	case 12: return batch_event_kernel<12>;
-	case 14: return batch_event_kernel<14>;
-	case 16: return batch_event_kernel<16>;
-	case 18: return batch_event_kernel<18>;
-	case 20: return batch_event_kernel<20>;
-	case 22: return batch_event_kernel<22>;
-	default: return batch_event_kernel<24>;
+	case 11: return batch_event_kernel<11>;
+	default: return batch_event_kernel<12>;
 	}
 }
 
@@ -759,8 +1022,9 @@ __global__ __launch_bounds__(256) void batch_plan_kernel(const BatchPlanArgs a)
 		if ((int)lane >= nRun)
 			a.colMap[(size_t)b * kCols + lane] = -1;
 		if (lane == 0) {
-			const uint32_t groups = (uint32_t)(nRun + kGroup - 1) / kGroup;
-			a.unitCount[b] = groups * (a.binChunk0[b + 1] - a.binChunk0[b]);
+			// a unit of a chunk covers up to four half groups
+			const uint32_t halves = (uint32_t)(nRun + kHalf - 1) / kHalf;
+			a.unitCount[b] = (halves + 3) / 4 * (a.binChunk0[b + 1] - a.binChunk0[b]);
 			count += a.evalAll ? 0 : nRun;
 		}
 	}
@@ -794,15 +1058,16 @@ __global__ __launch_bounds__(256) void batch_plan_kernel(const BatchPlanArgs a)
 	if (threadIdx.x == 0)
 		*a.nUnits = carry;
 	__syncthreads();
-	// the units of bin b (a wave per bin): chunk-major, column group minor
+	// the units of bin b (a wave per bin), chunk-major: four half groups each, the
+	// last of a chunk what remains (three or four: one per wave; fewer: shared)
 	for (uint32_t b = wv; b < a.nBins; b += kPlanWaves) {
 		const uint32_t off = a.unitCount[b];
-		const uint32_t n = (b + 1 < a.nBins ? a.unitCount[b + 1] : carry) - off;
-		const uint32_t chunks = a.binChunk0[b + 1] - a.binChunk0[b];
-		const uint32_t groups = chunks ? n / chunks : 0;
+		const uint32_t nRun = (uint32_t)__popcll(__ballot(a.startCol[(size_t)b * kCols + lane] >= 0));
+		const uint32_t halves = (nRun + kHalf - 1) / kHalf, per = (halves + 3) / 4;
+		const uint32_t n = per * (a.binChunk0[b + 1] - a.binChunk0[b]);
 		for (uint32_t k = lane; k < n; k += 64) {
-			const uint32_t c = k / groups, g = k % groups;
-			a.units[off + k] = (a.binChunk0[b] + c) * 4 + g;
+			const uint32_t c = k / per, first = 4 * (k % per);
+			a.units[off + k] = (a.binChunk0[b] + c) * 16 + first + (halves - first > 2 ? kFull : 0u);
 		}
 	}
 }
@@ -833,23 +1098,28 @@ __global__ __launch_bounds__(64) void batch_init_kernel(const BatchInitArgs a)
 		write_trial(a.st.xt + fit * a.P, a.W, a.P, a.T32 + fit * a.rowLen, a.flat2 + fit);
 }
 
-// complex128 [N][W] -> scaled complex64 [tiles * 32][rowLen] (zero padding)
-__global__ void batch_transform_kernel(const double2* __restrict__ src, uint64_t nEvents, uint32_t W,
-                                       uint32_t Wp, uint64_t nRows, const double* __restrict__ scale,
-                                       float2* __restrict__ dst)
+// complex128 [N][W] -> scaled complex64 in the permuted tile layout, [tiles][32]
+// [rowLen] floats (zero padding).  One thread per 16-byte unit of a row.
+__global__ __launch_bounds__(256) void batch_transform_kernel(const double* __restrict__ src, uint64_t nEvents,
+                                                              uint32_t W, uint32_t ks, uint64_t nRows,
+                                                              const double* __restrict__ scale,
+                                                              char* __restrict__ dst)
 {
 	const uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (idx >= nRows * Wp)
+	const uint32_t units = 4 * ks;
+	if (idx >= nRows * units)
 		return;
-	const uint64_t e = idx / Wp;
-	const uint32_t w = (uint32_t)(idx % Wp);
-	float2 out = make_float2(0.f, 0.f);
-	if (e < nEvents && w < W) {
-		const double2 v = src[e * W + w];
-		const double f = scale[w];
-		out = make_float2((float)(v.x * f), (float)(v.y * f));
+	const uint64_t e = idx / units;
+	const uint32_t u = (uint32_t)(idx % units);
+	f32x4 out = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+	for (uint32_t i = 0; i < 4; ++i) {
+		const uint32_t c = 16 * (u >> 2) + comp_of(u & 3, i);
+		if (e < nEvents && c / 2 < W)
+			out[i] = (float)(src[2 * e * W + c] * scale[c / 2]);
 	}
-	dst[idx] = out;
+	const uint32_t row = (uint32_t)(e % kEv);
+	*reinterpret_cast<f32x4*>(dst + e / kEv * tile_bytes(ks) + (size_t)row * (64 * ks) + 16 * (u ^ swizzle(ks, row))) = out;
 }
 
 uint64_t splitmix64(uint64_t x)
@@ -874,7 +1144,7 @@ struct rpwa_batch {
 	struct Bin {
 		uint64_t nEvents = 0;
 		uint32_t nTiles = 0;
-		float* d_amps = nullptr;
+		char* d_amps = nullptr;  // [tiles][32][rowLen] floats, permuted
 		std::vector<double> acc;  // [W][W] complex, normalised
 		double totAcc = 1.;
 	};
@@ -884,7 +1154,7 @@ struct rpwa_batch {
 	uint64_t totalEvents = 0;
 	uint64_t lastEvaluations = 0;
 	// device
-	float** d_binAmps = nullptr;
+	char** d_binAmps = nullptr;
 	uint32_t* d_chunkBin = nullptr;
 	uint32_t* d_chunkTile0 = nullptr;
 	uint32_t* d_binChunk0 = nullptr;
@@ -986,8 +1256,8 @@ BatchReduceArgs reduce_args(const rpwa_batch* b)
 
 int launch_event(rpwa_batch* b)
 {
-	hipLaunchKernelGGL(pick_event_kernel((int)(b->Wp / 4)), dim3(b->nWg), dim3(kThreads), 0, b->stream,
-	                   event_args(b));
+	const uint32_t ks = b->rowLen / 16;
+	hipLaunchKernelGGL(pick_event_kernel(ks), dim3(b->nWg), dim3(kThreads), event_lds(ks), b->stream, event_args(b));
 	RPWA_HIP_CHECK(hipGetLastError());
 	return RPWA_OK;
 }
@@ -1235,9 +1505,10 @@ extern "C" int rpwa_batch_add_bin(rpwa_batch* b, const double* amps, uint64_t nm
 		}
 	RPWA_HIP_CHECK(hipSetDevice(b->device));
 	const uint64_t nRows = (uint64_t)bin.nTiles * kEv;
-	RPWA_HIP_CHECK(hipMalloc(&bin.d_amps, nRows * b->rowLen * sizeof(float)));
+	const uint32_t ks = b->rowLen / 16;
+	RPWA_HIP_CHECK(hipMalloc(&bin.d_amps, (size_t)bin.nTiles * tile_bytes(ks)));
 	double* d_scale = nullptr;
-	double2* d_src = nullptr;
+	double* d_src = nullptr;
 	int rc = RPWA_OK;
 	do {
 		if (hipMalloc(&d_scale, W * sizeof(double)) != hipSuccess ||
@@ -1245,7 +1516,7 @@ extern "C" int rpwa_batch_add_bin(rpwa_batch* b, const double* amps, uint64_t nm
 			rc = RPWA_ERR_HIP;
 			break;
 		}
-		const double2* src = reinterpret_cast<const double2*>(amps);
+		const double* src = amps;
 		if (!onDevice) {
 			if (hipMalloc(&d_src, nmbEvents * W * sizeof(double2)) != hipSuccess ||
 			    hipMemcpy(d_src, amps, nmbEvents * W * sizeof(double2), hipMemcpyHostToDevice) != hipSuccess) {
@@ -1254,9 +1525,9 @@ extern "C" int rpwa_batch_add_bin(rpwa_batch* b, const double* amps, uint64_t nm
 			}
 			src = d_src;
 		}
-		const uint64_t n = nRows * b->Wp;
+		const uint64_t n = nRows * 4 * ks;
 		hipLaunchKernelGGL(batch_transform_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, b->stream, src,
-		                   nmbEvents, W, b->Wp, nRows, d_scale, reinterpret_cast<float2*>(bin.d_amps));
+		                   nmbEvents, W, ks, nRows, d_scale, bin.d_amps);
 		if (hipGetLastError() != hipSuccess || hipStreamSynchronize(b->stream) != hipSuccess)
 			rc = RPWA_ERR_HIP;
 	} while (false);
@@ -1290,7 +1561,7 @@ extern "C" int rpwa_batch_finish(rpwa_batch* b)
 	const uint32_t nBins = (uint32_t)b->bins.size();
 	// work chunks: each bin's tiles in runs of kChunkTiles
 	std::vector<uint32_t> binChunk0(nBins + 1, 0), nEv(nBins), chunkBin, chunkTile0;
-	std::vector<float*> ampPtr(nBins);
+	std::vector<char*> ampPtr(nBins);
 	std::vector<double> acc, totAcc(nBins);
 	b->nTiles = 0;
 	for (uint32_t i = 0; i < nBins; ++i) {
@@ -1309,8 +1580,8 @@ extern "C" int rpwa_batch_finish(rpwa_batch* b)
 	}
 	b->nChunks = binChunk0[nBins];
 	int occ = 0;
-	RPWA_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, pick_event_kernel((int)(b->Wp / 4)), kThreads,
-	                                                            0));
+	const uint32_t ks = b->rowLen / 16;
+	RPWA_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, pick_event_kernel(ks), kThreads, event_lds(ks)));
 	b->maxWgPerCu = (uint32_t)std::max(1, std::min(occ, 4));
 	const size_t F = nFits(b), slots = (size_t)b->nChunks * 4;
 	RPWA_TRY(dalloc(b, &b->d_binAmps, nBins));
@@ -1335,7 +1606,7 @@ extern "C" int rpwa_batch_finish(rpwa_batch* b)
 	RPWA_TRY(dalloc(b, &b->st.xt, F * b->P));
 	RPWA_TRY(dalloc(b, &b->st.gt, F * b->P));
 	RPWA_TRY(dalloc(b, &b->st.ft, F));
-	RPWA_HIP_CHECK(hipMemcpy(b->d_binAmps, ampPtr.data(), nBins * sizeof(float*), hipMemcpyHostToDevice));
+	RPWA_HIP_CHECK(hipMemcpy(b->d_binAmps, ampPtr.data(), nBins * sizeof(char*), hipMemcpyHostToDevice));
 	RPWA_HIP_CHECK(hipMemcpy(b->d_chunkBin, chunkBin.data(), b->nChunks * sizeof(uint32_t), hipMemcpyHostToDevice));
 	RPWA_HIP_CHECK(hipMemcpy(b->d_chunkTile0, chunkTile0.data(), b->nChunks * sizeof(uint32_t),
 	                         hipMemcpyHostToDevice));

@@ -7,17 +7,12 @@
 //   C = sum_e wt_e x_e x_e^T                      (D x D)
 // holds every product:
 //   Re I_ij = C[2i][2j] + C[2i+1][2j+1],   Im I_ij = C[2i+1][2j] - C[2i][2j+1].
-// C is computed as a rank-k update on v_mfma_f64_16x16x4_f64: 16x16 output
-// tiles of the upper triangle (tile row <= tile column), k = events.
-// A persistent grid of one 512-thread workgroup (8 waves) per CU walks event chunks
-// (grid-stride); each chunk is staged once through LDS and every wave issues
-// the MFMAs of its tiles from it.  Rows of up to 192 doubles (96 waves) take the
-// grouped kernel (tile map fixed at compile time, operand blocks read once per
-// step, pairs of waves splitting the steps); wider rows take windowed passes of
-// the same scheme over column windows of 8 blocks.  Each workgroup writes its
-// tile sums to a partial row; partial rows are summed in fixed order
-// (column_sum_kernel), and the host assembles the complex matrix.
+// C is computed as a rank-k update on v_mfma_f64_16x16x4_f64 (rank_update.h): 16x16
+// output tiles of the upper triangle (tile row <= tile column), k = events.  Each
+// workgroup writes its tile sums to a partial row; partial rows are summed in
+// fixed order (column_sum_kernel), and the host assembles the complex matrix.
 #include "internal.h"
+#include "rank_update.h"
 
 #include <algorithm>
 #include <cmath>
@@ -28,478 +23,6 @@
 
 namespace rpwa_amd {
 namespace {
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-
-constexpr int kIntThreads = 512;
-
-struct IntArgs {
-	const double* x;       // [M][D] row-major (interleaved complex rows)
-	const double* w;       // importance weights [M] or null (weight = 1/w)
-	uint64_t M;
-	uint32_t D;            // 2W
-	uint32_t Dp;           // D padded to a multiple of 16
-	uint32_t ldsStride;    // doubles per LDS row
-	uint32_t nT;           // Dp / 16
-	uint32_t nTiles;       // nT (nT + 1) / 2
-	uint32_t tileBase;     // windowed kernel: the pass index (the first pass writes the weight sums)
-	uint32_t winCol0;      // windowed kernel: first column (double) of the row window
-	uint32_t winCol1;      // windowed kernel: first column of the column window (off-diagonal pass)
-	uint32_t winI0;        // windowed kernel: first column block of the row window
-	uint32_t winJ0;        // windowed kernel: first column block of the column window
-	double* partials;      // [nWg][nTiles][256]
-	double* wsum;          // [nWg] sum of weights (1/w), or null
-	int accumulate;        // add to the existing partials
-	int directWeights;     // weight = w[e] instead of 1/w[e]
-};
-
-// ---------------------------------------------------------------------------
-// Grouped kernel for rows of up to 16 kGrpMaxBlocks doubles (NTB column blocks
-// of 16, row padded to Dp = 16 NTB).  The tile -> column-block map is fixed at
-// compile time, so a wave reads each 16-column operand block its tiles need once
-// per 4-event step and keeps it in registers (at most NTB LDS reads for up to
-// 20 MFMAs, instead of two reads per MFMA).  The upper-triangle tiles are split
-// into four contiguous groups of near-equal size, one per pair of waves
-// {g, g + 4}; the two waves of a pair take alternate 4-event steps of every
-// chunk, so no wave computes a dummy tile.  At the end the second wave of a
-// pair hands its sums to the first through LDS, in rounds that every wave runs
-// (same barriers), and the first writes the pair's sum (fixed order).
-constexpr int kGrpMaxBlocks = 12;
-constexpr int kLdsBytes = 160 * 1024;
-
-constexpr int tri_row(int nT, int t)
-{
-	int i = 0;
-	while (t >= nT - i) {
-		t -= nT - i;
-		++i;
-	}
-	return i;
-}
-constexpr int tri_col(int nT, int t) { return t - (tri_row(nT, t) * nT - tri_row(nT, t) * (tri_row(nT, t) - 1) / 2) + tri_row(nT, t); }
-constexpr int grp_begin(int nT, int g) { return g * (nT * (nT + 1) / 2) / 4; }
-constexpr int grp_size(int nT, int g) { return grp_begin(nT, g + 1) - grp_begin(nT, g); }
-constexpr int grp_max(int nT) { return (nT * (nT + 1) / 2 + 3) / 4; }
-// column blocks read by the tiles of group g: as A (rows) or as either operand
-constexpr uint32_t grp_blocks(int nT, int g, bool rowsOnly)
-{
-	uint32_t m = 0;
-	for (int t = grp_begin(nT, g); t < grp_begin(nT, g + 1); ++t) {
-		m |= 1u << tri_row(nT, t);
-		if (!rowsOnly)
-			m |= 1u << tri_col(nT, t);
-	}
-	return m;
-}
-// events per chunk: the largest multiple of 8 (up to 64) whose two LDS buffers,
-// [CH][Dp + 1] rows plus CH weights each, fit beside the 64 weight partials
-constexpr int grp_chunk(int nT)
-{
-	const int ch = (kLdsBytes - 64 * 8) / (2 * 8 * (16 * nT + 2)) / 8 * 8;
-	return ch < 64 ? ch : 64;
-}
-constexpr int grp_lds_doubles(int nT) { return 2 * grp_chunk(nT) * (16 * nT + 2); }
-// tiles per hand-over round: four groups' worth must fit in the chunk buffers
-constexpr int grp_round(int nT)
-{
-	const int r = grp_lds_doubles(nT) / (4 * 256);
-	return r < grp_max(nT) ? r : grp_max(nT);
-}
-
-template <int NT, int T>
-struct TileRC {
-	static constexpr int r = tri_row(NT, T);
-	static constexpr int c = tri_col(NT, T);
-};
-
-// one 4-event step of group G: read the group's operand blocks from the LDS row
-// xr (already offset by the lane's column), then one MFMA per tile
-template <int NTB, int G, bool WT, int... Q>
-__device__ __forceinline__ void grp_step(const double* __restrict__ xr, double wt, d4* acc,
-                                         std::integer_sequence<int, Q...>)
-{
-	constexpr int t0 = grp_begin(NTB, G);
-	constexpr uint32_t used = grp_blocks(NTB, G, false);
-	constexpr uint32_t rows = grp_blocks(NTB, G, true);
-	double v[NTB], va[NTB];
-#pragma unroll
-	for (int b = 0; b < NTB; ++b)
-		v[b] = (used >> b & 1) ? xr[16 * b] : 0.;
-#pragma unroll
-	for (int b = 0; b < NTB; ++b)
-		va[b] = (WT && (rows >> b & 1)) ? v[b] * wt : v[b];
-	((acc[Q] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[TileRC<NTB, t0 + Q>::r], v[TileRC<NTB, t0 + Q>::c], acc[Q],
-	                                                 0, 0, 0)),
-	 ...);
-}
-
-template <int NTB, bool WEIGHTED, int G>
-__device__ __forceinline__ void grp_body(const IntArgs& a, double* lds, double* wsh)
-{
-	constexpr int CH = grp_chunk(NTB);
-	// doubles per LDS row (16 NTB + 1) and per chunk buffer (rows, then weights); as
-	// run-time values the kernel measured 3% faster at 11 blocks than with them folded
-	const uint32_t STRIDE = a.ldsStride;
-	const uint32_t BUF = CH * STRIDE + CH;
-	constexpr int KL = (CH * 16 * NTB / 2 + kIntThreads - 1) / kIntThreads;  // double2 loads per thread
-	constexpr int NG = grp_size(NTB, G);
-	constexpr int kMaxG = grp_max(NTB);
-	constexpr int R = grp_round(NTB);
-	static_assert(CH % 8 == 0 && R >= 1, "chunk of whole step pairs, hand-over round of a tile at least");
-	const int tid = threadIdx.x;
-	const int lane = tid & 63;
-	const int h = tid >> 8;     // which wave of the pair (waves 0-3 or 4-7)
-	const int li = lane & 15;
-	const int lk = lane >> 4;
-
-	d4 acc[NG > 0 ? NG : 1];
-#pragma unroll
-	for (int q = 0; q < NG; ++q)
-		acc[q] = d4{0., 0., 0., 0.};
-
-	const uint32_t chunkD2 = CH * a.D / 2;
-	uint32_t ldsOff[KL];
-#pragma unroll
-	for (int l = 0; l < KL; ++l) {
-		const uint32_t idx = 2 * ((uint32_t)tid + (uint32_t)l * kIntThreads);
-		ldsOff[l] = (idx / a.D) * STRIDE + idx % a.D;
-	}
-	// padding columns (D..Dp) of both buffers stay zero
-	for (uint32_t i = tid; i < 2 * BUF; i += kIntThreads)
-		lds[i] = 0.;
-	__syncthreads();
-
-	double wacc = 0.;
-	const uint64_t nChunks = (a.M + CH - 1) / CH;
-	double2 stage[KL];
-	double wstage = 0.;
-	auto load_chunk = [&](uint64_t c) {
-		const uint64_t e0 = c * CH;
-		const uint64_t nEv = a.M - e0 < (uint64_t)CH ? a.M - e0 : (uint64_t)CH;
-		const uint32_t lim = (uint32_t)nEv * a.D / 2;
-		const double2* src = reinterpret_cast<const double2*>(a.x + e0 * a.D);
-#pragma unroll
-		for (int l = 0; l < KL; ++l) {
-			const uint32_t i2 = (uint32_t)tid + (uint32_t)l * kIntThreads;
-			stage[l] = (i2 < lim) ? src[i2] : make_double2(0., 0.);
-		}
-		if (tid < CH) {
-			const uint64_t e = e0 + tid;
-			wstage = e < a.M ? (a.w ? (a.directWeights ? a.w[e] : 1. / a.w[e]) : 1.) : 0.;
-		}
-	};
-	auto store_chunk = [&](int buf) {
-		double* xs = lds + buf * BUF;
-#pragma unroll
-		for (int l = 0; l < KL; ++l) {
-			const uint32_t i2 = (uint32_t)tid + (uint32_t)l * kIntThreads;
-			if (i2 < chunkD2) {
-				xs[ldsOff[l]] = stage[l].x;
-				xs[ldsOff[l] + 1] = stage[l].y;
-			}
-		}
-		if (tid < CH) {
-			xs[CH * STRIDE + tid] = wstage;
-			wacc += wstage;
-		}
-	};
-
-	uint64_t c = blockIdx.x;
-	int buf = 0;
-	if (c < nChunks) {
-		load_chunk(c);
-		store_chunk(0);
-	}
-	__syncthreads();
-	for (; c < nChunks; c += gridDim.x) {
-		const uint64_t next = c + gridDim.x;
-		if (next < nChunks)
-			load_chunk(next);  // in flight while the MFMAs below run
-		const double* xs = lds + buf * BUF;
-		const double* wts = xs + CH * STRIDE;
-		// not unrolled: unrolled, the steps' operand reads are hoisted together (more
-		// registers, 4% slower at 11 blocks)
-#pragma unroll 1
-		for (int kk = 0; kk < CH / 8; ++kk) {
-			const int row = (2 * kk + h) * 4 + lk;
-			const double wt = WEIGHTED ? wts[row] : 1.;
-			grp_step<NTB, G, WEIGHTED>(xs + row * STRIDE + li, wt, acc, std::make_integer_sequence<int, NG>{});
-		}
-		if (next < nChunks)
-			store_chunk(buf ^ 1);
-		__syncthreads();
-		buf ^= 1;
-	}
-
-	// hand-over: [group][tile of the round][register][lane] in the chunk buffers;
-	// v_mfma_f64_16x16x4_f64 leaves D[i][j] in lane j + 16 (i % 4), register i / 4
-	double* red = lds + G * R * 256;
-	double* out = a.partials + (size_t)blockIdx.x * a.nTiles * 256;
-#pragma unroll
-	for (int r0 = 0; r0 < kMaxG; r0 += R) {
-		if (h == 1) {
-#pragma unroll
-			for (int q = r0; q < NG && q < r0 + R; ++q)
-#pragma unroll
-				for (int v = 0; v < 4; ++v)
-					red[((q - r0) * 4 + v) * 64 + lane] = acc[q][v];
-		}
-		__syncthreads();
-		if (h == 0) {
-#pragma unroll
-			for (int q = r0; q < NG && q < r0 + R; ++q) {
-				double* o = out + (size_t)(grp_begin(NTB, G) + q) * 256;
-#pragma unroll
-				for (int v = 0; v < 4; ++v) {
-					const int i = lk + 4 * v;
-					double val = acc[q][v] + red[((q - r0) * 4 + v) * 64 + lane];
-					if (a.accumulate)
-						val += o[i * 16 + li];
-					o[i * 16 + li] = val;
-				}
-			}
-		}
-		__syncthreads();
-	}
-	if (tid < CH)
-		wsh[tid] = wacc;
-	__syncthreads();
-	if (a.wsum && tid == 0) {
-		double s = 0.;
-		for (int r = 0; r < CH; ++r)
-			s += wsh[r];
-		a.wsum[blockIdx.x] = a.accumulate ? a.wsum[blockIdx.x] + s : s;
-	}
-}
-
-template <int NTB, bool WEIGHTED>
-__global__ __launch_bounds__(kIntThreads) void integral_grp_kernel(IntArgs a)
-{
-	extern __shared__ double lds[];
-	__shared__ double wsh[64];
-	// wave-uniform branch: waves g and g + 4 run group g
-	switch ((threadIdx.x >> 6) & 3) {
-	case 0: grp_body<NTB, WEIGHTED, 0>(a, lds, wsh); break;
-	case 1: grp_body<NTB, WEIGHTED, 1>(a, lds, wsh); break;
-	case 2: grp_body<NTB, WEIGHTED, 2>(a, lds, wsh); break;
-	default: grp_body<NTB, WEIGHTED, 3>(a, lds, wsh); break;
-	}
-}
-
-// ---------------------------------------------------------------------------
-// Windowed passes for rows wider than 16 kGrpMaxBlocks doubles (the Hessian's
-// derivative rows): the column blocks are cut into windows of kWin; a pass
-// stages only its windows' columns of every row (one window for a diagonal
-// pass, the kWin (kWin + 1) / 2 tiles of its triangle; two windows for an
-// off-diagonal pass, the kWin x kWin tiles between them) and computes its tiles
-// with the grouped kernel's scheme (compile-time tile map, operand blocks read
-// once per step, pairs of waves splitting the steps).  Blocks past the row
-// (the last window's padding) are staged as zeros and their tiles not written.
-constexpr int kWin = 8;
-
-constexpr int win_blocks_of(bool rect) { return rect ? 2 * kWin : kWin; }
-constexpr int win_tiles(bool rect) { return rect ? kWin * kWin : kWin * (kWin + 1) / 2; }
-constexpr int win_row(bool rect, int t) { return rect ? t / kWin : tri_row(kWin, t); }
-constexpr int win_col(bool rect, int t) { return rect ? kWin + t % kWin : tri_col(kWin, t); }
-constexpr int win_begin(bool rect, int g) { return g * win_tiles(rect) / 4; }
-constexpr int win_size(bool rect, int g) { return win_begin(rect, g + 1) - win_begin(rect, g); }
-constexpr int win_max(bool rect) { return (win_tiles(rect) + 3) / 4; }
-constexpr uint32_t win_blocks(bool rect, int g, bool rowsOnly)
-{
-	uint32_t m = 0;
-	for (int t = win_begin(rect, g); t < win_begin(rect, g + 1); ++t) {
-		m |= 1u << win_row(rect, t);
-		if (!rowsOnly)
-			m |= 1u << win_col(rect, t);
-	}
-	return m;
-}
-constexpr int win_chunk(bool rect)
-{
-	const int ch = (kLdsBytes - 64 * 8) / (2 * 8 * (16 * win_blocks_of(rect) + 2)) / 8 * 8;
-	return ch < 64 ? ch : 64;
-}
-constexpr int win_lds_doubles(bool rect) { return 2 * win_chunk(rect) * (16 * win_blocks_of(rect) + 2); }
-
-template <bool RECT, int T>
-struct WinRC {
-	static constexpr int r = win_row(RECT, T);
-	static constexpr int c = win_col(RECT, T);
-};
-
-template <bool RECT, int G, bool WT, int... Q>
-__device__ __forceinline__ void win_step(const double* __restrict__ xr, double wt, d4* acc,
-                                         std::integer_sequence<int, Q...>)
-{
-	constexpr int NB = win_blocks_of(RECT);
-	constexpr int t0 = win_begin(RECT, G);
-	constexpr uint32_t used = win_blocks(RECT, G, false);
-	constexpr uint32_t rows = win_blocks(RECT, G, true);
-	double v[NB], va[NB];
-#pragma unroll
-	for (int b = 0; b < NB; ++b)
-		v[b] = (used >> b & 1) ? xr[16 * b] : 0.;
-#pragma unroll
-	for (int b = 0; b < NB; ++b)
-		va[b] = (WT && (rows >> b & 1)) ? v[b] * wt : v[b];
-	((acc[Q] = __builtin_amdgcn_mfma_f64_16x16x4f64(va[WinRC<RECT, t0 + Q>::r], v[WinRC<RECT, t0 + Q>::c], acc[Q],
-	                                                 0, 0, 0)),
-	 ...);
-}
-
-template <bool RECT, bool WEIGHTED, int G>
-__device__ __forceinline__ void win_body(const IntArgs& a, double* lds, double* wsh)
-{
-	constexpr int CH = win_chunk(RECT);
-	constexpr int WS = 16 * win_blocks_of(RECT);       // staged doubles per row
-	constexpr int W0 = 16 * kWin;                      // doubles of the row window
-	constexpr int KL = CH * WS / 2 / kIntThreads;      // double2 loads per thread (exact)
-	constexpr int NG = win_size(RECT, G);
-	constexpr int kMaxG = win_max(RECT);
-	static_assert(CH * WS / 2 == KL * kIntThreads && CH % 8 == 0, "chunk of whole loads and step pairs");
-	static_assert(win_lds_doubles(RECT) >= 4 * kMaxG * 256, "hand-over in one round");
-	// LDS row stride (WS + 1) as a run-time value, as in the grouped kernel
-	const uint32_t STRIDE = a.ldsStride;
-	const uint32_t BUF = CH * STRIDE + CH;
-	const int tid = threadIdx.x;
-	const int lane = tid & 63;
-	const int h = tid >> 8;
-	const int li = lane & 15;
-	const int lk = lane >> 4;
-
-	d4 acc[NG];
-#pragma unroll
-	for (int q = 0; q < NG; ++q)
-		acc[q] = d4{0., 0., 0., 0.};
-
-	// staging geometry: double2 number tid + 512 l of the chunk's staged block is
-	// column k of event e of the block; its source column g in the row
-	uint32_t ldsOff[KL], srcOff[KL], srcEv[KL];
-	bool colOk[KL];
-#pragma unroll
-	for (int l = 0; l < KL; ++l) {
-		const uint32_t i2 = (uint32_t)tid + (uint32_t)l * kIntThreads;
-		const uint32_t e = i2 / (WS / 2), k = 2 * (i2 % (WS / 2));
-		const uint32_t g = k < (uint32_t)W0 ? a.winCol0 + k : a.winCol1 + (k - W0);
-		ldsOff[l] = e * STRIDE + k;
-		srcOff[l] = e * a.D + g;
-		srcEv[l] = e;
-		colOk[l] = g < a.D;
-	}
-	for (uint32_t i = tid; i < 2 * BUF; i += kIntThreads)
-		lds[i] = 0.;
-	__syncthreads();
-
-	double wacc = 0.;
-	const uint64_t nChunks = (a.M + CH - 1) / CH;
-	double2 stage[KL];
-	double wstage = 0.;
-	auto load_chunk = [&](uint64_t c) {
-		const uint64_t e0 = c * CH;
-		const uint64_t nEv = a.M - e0 < (uint64_t)CH ? a.M - e0 : (uint64_t)CH;
-		const double* src = a.x + e0 * a.D;
-#pragma unroll
-		for (int l = 0; l < KL; ++l)
-			stage[l] = (colOk[l] && srcEv[l] < (uint32_t)nEv) ? *reinterpret_cast<const double2*>(src + srcOff[l])
-			                                                  : make_double2(0., 0.);
-		if (tid < CH) {
-			const uint64_t e = e0 + tid;
-			wstage = e < a.M ? (a.w ? (a.directWeights ? a.w[e] : 1. / a.w[e]) : 1.) : 0.;
-		}
-	};
-	auto store_chunk = [&](int buf) {
-		double* xs = lds + buf * BUF;
-#pragma unroll
-		for (int l = 0; l < KL; ++l) {
-			xs[ldsOff[l]] = stage[l].x;
-			xs[ldsOff[l] + 1] = stage[l].y;
-		}
-		if (tid < CH) {
-			xs[CH * STRIDE + tid] = wstage;
-			wacc += wstage;
-		}
-	};
-
-	uint64_t c = blockIdx.x;
-	int buf = 0;
-	if (c < nChunks) {
-		load_chunk(c);
-		store_chunk(0);
-	}
-	__syncthreads();
-	for (; c < nChunks; c += gridDim.x) {
-		const uint64_t next = c + gridDim.x;
-		if (next < nChunks)
-			load_chunk(next);
-		const double* xs = lds + buf * BUF;
-		const double* wts = xs + CH * STRIDE;
-#pragma unroll 1
-		for (int kk = 0; kk < CH / 8; ++kk) {
-			const int row = (2 * kk + h) * 4 + lk;
-			const double wt = WEIGHTED ? wts[row] : 1.;
-			win_step<RECT, G, WEIGHTED>(xs + row * STRIDE + li, wt, acc, std::make_integer_sequence<int, NG>{});
-		}
-		if (next < nChunks)
-			store_chunk(buf ^ 1);
-		__syncthreads();
-		buf ^= 1;
-	}
-
-	// hand-over as in the grouped kernel (one round), then the pair's sums go to
-	// their tiles of the full triangle (padding tiles past the row are dropped)
-	double* red = lds + G * kMaxG * 256;
-	double* out = a.partials + (size_t)blockIdx.x * a.nTiles * 256;
-	if (h == 1) {
-#pragma unroll
-		for (int q = 0; q < NG; ++q)
-#pragma unroll
-			for (int v = 0; v < 4; ++v)
-				red[(q * 4 + v) * 64 + lane] = acc[q][v];
-	}
-	__syncthreads();
-	if (h == 0) {
-#pragma unroll
-		for (int q = 0; q < NG; ++q) {
-			const int t = win_begin(RECT, G) + q;
-			const uint32_t I = a.winI0 + win_row(RECT, t);
-			const uint32_t J = RECT ? a.winJ0 + (win_col(RECT, t) - kWin) : a.winI0 + win_col(RECT, t);
-			if (J >= a.nT)
-				continue;
-			double* o = out + (size_t)(I * a.nT - I * (I - 1) / 2 + (J - I)) * 256;
-#pragma unroll
-			for (int v = 0; v < 4; ++v) {
-				const int i = lk + 4 * v;
-				double val = acc[q][v] + red[(q * 4 + v) * 64 + lane];
-				if (a.accumulate)
-					val += o[i * 16 + li];
-				o[i * 16 + li] = val;
-			}
-		}
-	}
-	__syncthreads();
-	if (tid < CH)
-		wsh[tid] = wacc;
-	__syncthreads();
-	if (a.wsum && a.tileBase == 0 && tid == 0) {
-		double s = 0.;
-		for (int r = 0; r < CH; ++r)
-			s += wsh[r];
-		a.wsum[blockIdx.x] = a.accumulate ? a.wsum[blockIdx.x] + s : s;
-	}
-}
-
-template <bool RECT, bool WEIGHTED>
-__global__ __launch_bounds__(kIntThreads) void integral_win_kernel(IntArgs a)
-{
-	extern __shared__ double lds[];
-	__shared__ double wsh[64];
-	switch ((threadIdx.x >> 6) & 3) {
-	case 0: win_body<RECT, WEIGHTED, 0>(a, lds, wsh); break;
-	case 1: win_body<RECT, WEIGHTED, 1>(a, lds, wsh); break;
-	case 2: win_body<RECT, WEIGHTED, 2>(a, lds, wsh); break;
-	default: win_body<RECT, WEIGHTED, 3>(a, lds, wsh); break;
-	}
-}
 
 // fixed-order column sums of a [nRows][nCols] array
 constexpr int kColElems = 64;
@@ -529,112 +52,43 @@ __global__ __launch_bounds__(kColElems* kColChunks) void column_sum_kernel(
 
 }  // namespace
 
-typedef void (*IntKernel)(IntArgs);
-template <bool WT>
-static IntKernel pick_grp(uint32_t nT)
+hipError_t launch_column_sum(const double* in, int nRows, uint32_t nCols, double* out, hipStream_t s)
 {
-	switch (nT) {
-	case 1: return integral_grp_kernel<1, WT>;
-	case 2: return integral_grp_kernel<2, WT>;
-	case 3: return integral_grp_kernel<3, WT>;
-	case 4: return integral_grp_kernel<4, WT>;
-	case 5: return integral_grp_kernel<5, WT>;
-	case 6: return integral_grp_kernel<6, WT>;
-	case 7: return integral_grp_kernel<7, WT>;
-	case 8: return integral_grp_kernel<8, WT>;
-	case 9: return integral_grp_kernel<9, WT>;
-	case 10: return integral_grp_kernel<10, WT>;
-	case 11: return integral_grp_kernel<11, WT>;
-	case 12: return integral_grp_kernel<12, WT>;
-	default: return nullptr;
-	}
+	hipLaunchKernelGGL(column_sum_kernel, dim3((nCols + kColElems - 1) / kColElems), dim3(kColElems * kColChunks), 0, s,
+	                   in, nRows, nCols, out);
+	return hipGetLastError();
 }
-static int grp_chunk_of(uint32_t nT) { return grp_chunk((int)nT); }
+
+// partial tiles of n rows of D doubles (D even)
+static hipError_t launch_rows(const double* x, const double* w, bool direct, uint64_t n, uint32_t D, double* partials,
+                              double* wsum, bool accumulate, int nWg, hipStream_t s)
+{
+	ru::Args a{};
+	a.x = x;
+	a.w = w;
+	a.n = n;
+	a.D = D;
+	a.partials = partials;
+	a.wsum = wsum;
+	a.accumulate = accumulate ? 1 : 0;
+	a.direct = direct ? 1 : 0;
+	return w ? ru::launch<true>(a, nWg, s) : ru::launch<false>(a, nWg, s);
+}
 
 struct IntegralPlan {
-	uint32_t D, Dp, nT, nTiles, ldsStride;
-	int chunk;
+	uint32_t nT, nTiles;
 	int nWg;
-	size_t lds;
-	IntKernel kern = nullptr;  // grouped kernel (one pass over every tile)
-	// windowed passes (rows of more than 16 kGrpMaxBlocks doubles): diagonal and
-	// off-diagonal window kernels, their LDS row strides and dynamic LDS
-	bool windowed = false;
-	IntKernel kernDiag = nullptr, kernRect = nullptr;
-	uint32_t strideDiag = 0, strideRect = 0;
-	size_t ldsDiag = 0, ldsRect = 0;
 };
 
-// D = real row length (2 x complex values per row)
-static int integral_plan(int device, uint32_t D, bool weighted, IntegralPlan& p)
+// D = real row length (2 x complex values per row); one workgroup per CU
+static int integral_plan(int device, uint32_t D, IntegralPlan& p)
 {
-	p.D = D;
-	p.Dp = (p.D + 15) / 16 * 16;
-	p.nT = p.Dp / 16;
+	p.nT = (D + 15) / 16;
 	p.nTiles = p.nT * (p.nT + 1) / 2;
-	p.ldsStride = p.Dp + 1;  // odd stride spreads the 4 rows of a read over the banks
-	p.kern = weighted ? pick_grp<true>(p.nT) : pick_grp<false>(p.nT);
-	if (p.kern) {
-		p.chunk = grp_chunk_of(p.nT);
-		p.lds = 2 * ((size_t)p.chunk * p.ldsStride + p.chunk) * sizeof(double);
-	} else {
-		// wider rows (the Hessian's derivative rows): windowed passes
-		p.windowed = true;
-		p.kernDiag = weighted ? integral_win_kernel<false, true> : integral_win_kernel<false, false>;
-		p.kernRect = weighted ? integral_win_kernel<true, true> : integral_win_kernel<true, false>;
-		p.strideDiag = 16 * win_blocks_of(false) + 1;
-		p.strideRect = 16 * win_blocks_of(true) + 1;
-		p.ldsDiag = (size_t)win_lds_doubles(false) * sizeof(double);
-		p.ldsRect = (size_t)win_lds_doubles(true) * sizeof(double);
-		p.chunk = win_chunk(true);
-		p.lds = std::max(p.ldsDiag, p.ldsRect);
-	}
 	int nCu = 0;
 	RPWA_HIP_CHECK(hipDeviceGetAttribute(&nCu, hipDeviceAttributeMultiprocessorCount, device));
 	p.nWg = nCu > 0 ? nCu : 1;
 	return RPWA_OK;
-}
-
-// Launch the rank-k update's passes on stream s: one grouped launch, or the
-// windowed diagonal and off-diagonal passes (every tile of the triangle written
-// by exactly one pass).
-static hipError_t launch_plan(const IntegralPlan& p, IntArgs a, hipStream_t s)
-{
-	auto allow = [](IntKernel k, size_t lds) -> hipError_t {
-		// dynamic LDS beyond 64 KiB is requested explicitly
-		if (lds + 64 * sizeof(double) > 64u * 1024u)
-			return hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-			                           (int)lds);
-		return hipSuccess;
-	};
-	if (p.windowed) {
-		if (hipError_t e = allow(p.kernDiag, p.ldsDiag))
-			return e;
-		if (hipError_t e = allow(p.kernRect, p.ldsRect))
-			return e;
-		const uint32_t nWin = (p.nT + kWin - 1) / kWin;
-		uint32_t pass = 0;
-		for (uint32_t u = 0; u < nWin; ++u)
-			for (uint32_t v = u; v < nWin; ++v, ++pass) {
-				const bool rect = v > u;
-				a.tileBase = pass;
-				a.winI0 = u * kWin;
-				a.winJ0 = v * kWin;
-				a.winCol0 = 16 * u * kWin;
-				a.winCol1 = 16 * v * kWin;
-				a.ldsStride = rect ? p.strideRect : p.strideDiag;
-				hipLaunchKernelGGL(rect ? p.kernRect : p.kernDiag, dim3(p.nWg), dim3(kIntThreads),
-				                   rect ? p.ldsRect : p.ldsDiag, s, a);
-				if (hipError_t e = hipGetLastError())
-					return e;
-			}
-		return hipSuccess;
-	}
-	if (hipError_t e = allow(p.kern, p.lds))
-		return e;
-	a.tileBase = 0;
-	hipLaunchKernelGGL(p.kern, dim3(p.nWg), dim3(kIntThreads), p.lds, s, a);
-	return hipGetLastError();
 }
 
 // Per-device work area of the rank-k update (workgroup partial tiles, weight
@@ -686,7 +140,7 @@ int syrk_run(int device, const double* d_x, uint64_t M, uint32_t D, const double
 	RPWA_HIP_CHECK(hipSetDevice(device));
 	const bool weighted = (d_w != nullptr) || (h_w != nullptr);
 	IntegralPlan p;
-	int st = integral_plan(device, D, weighted, p);
+	int st = integral_plan(device, D, p);
 	if (st != RPWA_OK)
 		return st;
 	SyrkWork& work = syrk_work(device);
@@ -719,14 +173,8 @@ int syrk_run(int device, const double* d_x, uint64_t M, uint32_t D, const double
 	double* d_part = work.part;
 	double* d_wsum = work.wsum;
 	double* d_red = work.red;
-	// every pass re-reads the rows for its own set of output tiles
-	auto launch_passes = [&](IntArgs aa) -> hipError_t { return launch_plan(p, aa, s); };
-	IntArgs a;
-	a.D = p.D; a.Dp = p.Dp; a.ldsStride = p.ldsStride; a.nT = p.nT; a.nTiles = p.nTiles;
-	a.partials = d_part; a.wsum = d_wsum; a.directWeights = directWeights ? 1 : 0;
 	if (d_x) {
-		a.x = d_x; a.w = d_w; a.M = M; a.accumulate = 0;
-		INT_CHECK(launch_passes(a));
+		INT_CHECK(launch_rows(d_x, d_w, directWeights, M, D, d_part, d_wsum, false, p.nWg, s));
 	} else {
 		// stream the host array through two device buffers
 		const uint64_t chunkEv = std::max<uint64_t>(1, (256ull << 20) / (8ull * D));
@@ -747,9 +195,8 @@ int syrk_run(int device, const double* d_x, uint64_t M, uint32_t D, const double
 			INT_CHECK(hipMemcpyAsync(d_stage[b], h_x + off * D, n * 8ull * D, hipMemcpyHostToDevice, s));
 			if (weighted)
 				INT_CHECK(hipMemcpyAsync(d_wstage[b], h_w + off, n * sizeof(double), hipMemcpyHostToDevice, s));
-			a.x = d_stage[b]; a.w = weighted ? d_wstage[b] : nullptr; a.M = n;
-			a.accumulate = first ? 0 : 1;
-			INT_CHECK(launch_passes(a));
+			INT_CHECK(launch_rows(d_stage[b], weighted ? d_wstage[b] : nullptr, directWeights, n, D, d_part, d_wsum, !first,
+			                      p.nWg, s));
 			INT_CHECK(hipEventRecord(done[b], s));
 			first = false;
 		}
@@ -757,12 +204,10 @@ int syrk_run(int device, const double* d_x, uint64_t M, uint32_t D, const double
 		(void)hipEventDestroy(done[0]);
 		(void)hipEventDestroy(done[1]);
 	}
-	const int nb = (int)((p.nTiles * 256 + kColElems - 1) / kColElems);
-	hipLaunchKernelGGL(column_sum_kernel, dim3(nb), dim3(kColElems * kColChunks), 0, s, d_part, p.nWg,
-	                   p.nTiles * 256, d_red);
-	INT_CHECK(hipGetLastError());
+	INT_CHECK(launch_column_sum(d_part, p.nWg, p.nTiles * 256, d_red, s));
 	INT_CHECK(hipMemcpyAsync(C.data(), d_red, C.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-	INT_CHECK(hipMemcpyAsync(wsums.data(), d_wsum, wsums.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+	if (weighted)
+		INT_CHECK(hipMemcpyAsync(wsums.data(), d_wsum, wsums.size() * sizeof(double), hipMemcpyDeviceToHost, s));
 	INT_CHECK(hipStreamSynchronize(s));
 #undef INT_CHECK
 	// the symmetric matrix from the upper-triangle tiles, tile by tile: a
@@ -782,7 +227,7 @@ int syrk_run(int device, const double* d_x, uint64_t M, uint32_t D, const double
 				}
 		}
 	if (wtot) {
-		double t = 0.;
+		double t = weighted ? 0. : (double)M;
 		for (double v : wsums)
 			t += v;
 		*wtot = t;
@@ -973,27 +418,11 @@ static int integral_noalloc(int device, const double* d_amps, uint64_t M, uint32
 	double* const base = g_naPtr[device];
 	const bool weighted = d_w != nullptr;
 	IntegralPlan p;
-	if (int st = integral_plan(device, 2 * W, weighted, p))
+	if (int st = integral_plan(device, 2 * W, p))
 		return st;
 	p.nWg = std::min(p.nWg, kNaWg);
-	IntArgs a;
-	a.x = d_amps;
-	a.w = d_w;
-	a.M = M;
-	a.D = p.D;
-	a.Dp = p.Dp;
-	a.ldsStride = p.ldsStride;
-	a.nT = p.nT;
-	a.nTiles = p.nTiles;
-	a.partials = base;
-	a.wsum = base + kNaWsum;
-	a.accumulate = 0;
-	a.directWeights = 0;
-	RPWA_HIP_CHECK(launch_plan(p, a, 0));
-	const int nb = (int)((p.nTiles * 256 + kColElems - 1) / kColElems);
-	hipLaunchKernelGGL(column_sum_kernel, dim3(nb), dim3(kColElems * kColChunks), 0, 0, base, p.nWg,
-	                   p.nTiles * 256, base + kNaRed);
-	RPWA_HIP_CHECK(hipGetLastError());
+	RPWA_HIP_CHECK(launch_rows(d_amps, d_w, false, M, 2 * W, base, base + kNaWsum, false, p.nWg, 0));
+	RPWA_HIP_CHECK(launch_column_sum(base, p.nWg, p.nTiles * 256, base + kNaRed, 0));
 	hipLaunchKernelGGL(assemble_kernel, dim3((W * W + 255) / 256), dim3(256), 0, 0, base + kNaRed, p.nT, W,
 	                   base + kNaWsum, p.nWg, M, weighted ? 1 : 0, base + kNaOut);
 	RPWA_HIP_CHECK(hipGetLastError());

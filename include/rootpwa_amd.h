@@ -116,11 +116,12 @@ int rpwa_lik_collect(rpwa_lik_ctx* ctx, double* logLikelihood, double* derivativ
 /* Event part of the Hessian (pwaLikelihood.cc:697-753): for a, b over the
  * [rank][2][nmbWavesMax] production amplitudes, hessian[a][b][3] holds the
  * real/real, real/imag and imag/imag event sums; flatTerms[a] (complex) the
- * mixed flat-wave terms and hessianFlat the flat/flat term.  The per-event rows
- * live in a device work area shared by the calls on one GPU (serialised),
- * grown to the largest call and kept until the process ends: (nEvents or 8 GiB
- * worth of rows) x 16 (rank W + W + 2) bytes, 8.5 GB at 2M events x 345
- * parameters. */
+ * mixed flat-wave terms and hessianFlat the flat/flat term.  The per-event sums
+ * and the workgroups' partial sums live in a device work area shared by the calls
+ * on one GPU (serialised), grown to the largest call and kept until the process
+ * ends: (nEvents or 8 GiB worth) x 16 (2 rank + 1) bytes, and per CU 2 KB for
+ * every 16 x 16 tile of the triangles of 2 rank W and 2 W columns; 0.33 GB at 2M
+ * events x 88 waves x rank 2. */
 int rpwa_lik_hessian(rpwa_lik_ctx* ctx, const double* prodAmps, uint32_t nmbProdAmps,
                      double prodAmpFlat, uint32_t rank, double* hessian, double* flatTerms,
                      double* hessianFlat);

@@ -130,7 +130,7 @@ static hipError_t syrk_grow(double*& buf, size_t& cap, size_t need)
 // Weighted real rank-k update C = sum_e wt_e x_e x_e^T of M rows of D doubles
 // (device or host memory); wt_e = w[e] (directWeights) or 1/w[e] or 1.
 // Returns the full symmetric D x D matrix and the sum of the weights.
-int syrk_run(int device, const double* d_x, uint64_t M, uint32_t D, const double* d_w, bool directWeights,
+static int syrk_run(int device, const double* d_x, uint64_t M, uint32_t D, const double* d_w, bool directWeights,
              const double* h_x, const double* h_w, std::vector<double>& full, double* wtot)
 {
 	if (device < 0 || device >= kSyrkDevices) {

@@ -125,9 +125,6 @@ hipError_t launch_event_reduce(const double* partials, int nWg, uint32_t nElem, 
                                double* out, hipStream_t s,
                                unsigned long long* doneFlag = nullptr, unsigned long long seq = 0,
                                hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
-// weighted real rank-k update (integral.hip): full D x D matrix of sum_e wt_e x_e x_e^T
-int syrk_run(int device, const double* d_x, uint64_t M, uint32_t D, const double* d_w, bool directWeights,
-             const double* h_x, const double* h_w, std::vector<double>& full, double* wtot);
 // fixed-order column sums of a device array [nRows][nCols] (integral.hip)
 hipError_t launch_column_sum(const double* in, int nRows, uint32_t nCols, double* out, hipStream_t s);
 // *flag |= 1 if column `wave` of amps [nEvents][W] (complex128) has a non-zero element

@@ -28,3 +28,49 @@ def test_integral(gpu, waves, events):
     assert H.rel_err(gpu.integral(a), a.T @ a.conj()) <= 1e-12
     ref = (a / w[:, None]).T @ a.conj() * (events / np.sum(1 / w))
     assert H.rel_err(gpu.integral(a, w), ref) <= 1e-12
+
+
+def hessian(A, nW, T, flat):
+    """[P][P][3], [P], float of pwaLikelihood.cc:697-753 over P = rank 2 wmax amplitudes."""
+    rank, wmax = T.shape[0], T.shape[2]
+    W = sum(nW)
+    sec = (np.arange(W) >= nW[0]).astype(int)
+    at = np.where(sec, np.arange(W) - nW[0], np.arange(W))
+    S = np.stack([np.stack([A[:, sec == s] @ T[r, s, :nW[s]] for s in range(2)]) for r in range(rank)])
+    f = 2 / (np.sum(np.abs(S) ** 2, axis=(0, 1)) + flat ** 2)
+    h = np.zeros((rank, 2, wmax, rank, 2, wmax, 3))
+    ft = np.zeros((rank, 2, wmax), dtype=complex)
+    d = [f[:, None] * S[r][sec].T * A.conj() for r in range(rank)]
+    Q = (A * f[:, None]).T @ A.conj()
+    for r in range(rank):
+        ft[r, sec, at] = flat * f @ d[r]
+        for q in range(rank):
+            same = (sec[:, None] == sec[None, :]) & (r == q)
+            for k, v in enumerate((d[r].real.T @ d[q].real - same * Q.real, d[r].real.T @ d[q].imag - same * Q.imag,
+                                   d[r].imag.T @ d[q].imag - same * Q.real)):
+                for i in range(W):
+                    h[r, sec[i], at[i], q, sec, at, k] = v[i]
+    P = rank * 2 * wmax
+    return h.reshape(P, P, 3), ft, flat ** 2 * np.sum(f ** 2) - np.sum(f)
+
+
+@pytest.mark.parametrize("nW,rank,events", [((0, 1), 1, 1), ((7, 0), 1, 63), ((3, 5), 2, 65), ((2, 3), 5, 40),
+                                            ((8, 80), 1, 56), ((0, 96), 1, 300), ((1, 103), 1, 64),
+                                            ((0, 136), 1, 129), ((13, 40), 3, 1000), ((8, 80), 2, 64 * 256 * 2 + 9)])
+@pytest.mark.parametrize("prec", [0, 1], ids=["fp64", "mixed"])
+def test_hessian(gpu, nW, rank, events, prec):
+    rng = np.random.default_rng(sum(nW) + rank)
+    A = amplitudes(rng, events, sum(nW))
+    T = np.zeros((rank, 2, max(nW)), dtype=complex)
+    for s in range(2):
+        T[:, s, :nW[s]] = rng.normal(size=(rank, nW[s])) + 1j * rng.normal(size=(rank, nW[s]))
+    if prec:  # the stored amplitudes; everything after them is FP64
+        A = A.astype(np.complex64).astype(np.complex128)
+    ctx = gpu.LikelihoodContext(0, prec)
+    ctx.load(A, nW)
+    flat = 0.7
+    h, ft, hf = ctx.hessian(T, flat)
+    rh, rft, rhf = hessian(A, nW, T, flat)
+    assert H.rel_err(h, rh) <= 1e-12
+    assert H.rel_err(ft, rft) <= 1e-12
+    assert abs(hf - rhf) <= 1e-12 * abs(rhf) * 10  # a difference of two sums

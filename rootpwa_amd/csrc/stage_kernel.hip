@@ -995,6 +995,9 @@ __global__ __launch_bounds__(kThreads, 2) void wave_tile_kernel(StageArgs a)
 
 using StageKernel = void (*)(StageArgs);
 
+// rank 3 has its own instantiation: on rank 4's a quarter of the FP64 work of S and
+// of the gradient is spent on zeros (300k events x 53 waves x rank 3, complex64:
+// event kernel 53 -> 46 us)
 template <bool MIXED, int E, int NG>
 StageKernel pick_r(int rank)
 {
@@ -1002,6 +1005,8 @@ StageKernel pick_r(int rank)
 		return stage_kernel<MIXED, 1, E, NG>;
 	if (rank <= 2)
 		return stage_kernel<MIXED, 2, E, NG>;
+	if (rank <= 3)
+		return stage_kernel<MIXED, 3, E, NG>;
 	return stage_kernel<MIXED, 4, E, NG>;
 }
 
@@ -1065,7 +1070,7 @@ StageKernel pick_stage(const AmpLayout& lay, int events, int gm, int rank)
 
 }  // namespace
 
-int stage_rank_cap(int rank) { return rank <= 1 ? 1 : (rank <= 2 ? 2 : 4); }
+int stage_rank_cap(int rank) { return rank < 1 ? 1 : (rank < 4 ? rank : 4); }
 
 bool stage_t_inline(const AmpLayout& lay, int rank)
 {
@@ -1101,10 +1106,7 @@ bool stage_plan(const AmpLayout& lay, int events, int rank, StagePlan& p, int gm
 	p.rowUnitsP = p.rowUnits | 1u;
 	p.ranks = stage_rank_cap(rank);
 	const bool mixed = lay.precision == RPWA_PREC_MIXED;
-	const uint32_t ug = (uint32_t)(mixed ? (p.ranks == 1 ? group_units<true, 1>() : p.ranks == 2 ? group_units<true, 2>()
-	                                                                                     : group_units<true, 4>())
-	                                     : (p.ranks == 1 ? group_units<false, 1>() : p.ranks == 2 ? group_units<false, 2>()
-	                                                                                     : group_units<false, 4>()));
+	const uint32_t ug = (uint32_t)((mixed ? 2 : 1) * p.ranks <= 2 ? 4 : 2);  // group_units
 	const uint32_t secUnit = lay.secOff[1] * bpc / 16u;
 	p.gGroups0 = (secUnit + ug - 1) / ug;
 	p.gGroups = p.gGroups0 + (p.rowUnits - secUnit + ug - 1) / ug;
@@ -1112,7 +1114,7 @@ bool stage_plan(const AmpLayout& lay, int events, int rank, StagePlan& p, int gm
 		return false;
 	p.gSubs = (uint32_t)threads / p.gGroups;
 	p.stageBytes = ((uint32_t)events * p.rowUnitsP + 1u) * 16u;
-	const int ps = p.ranks == 1 ? part_stride<1>() : p.ranks == 2 ? part_stride<2>() : part_stride<4>();
+	const int ps = 2 * p.ranks + 1;  // part_stride
 	// S partials of waves 1..3 (u replaces wave 1's)
 	const size_t partBytes = (size_t)(waves - 1) * events * ps * sizeof(double2);
 	const size_t endBytes = (size_t)p.gSubs * p.rowUnits * P * p.ranks * sizeof(double2) +
@@ -1121,7 +1123,7 @@ bool stage_plan(const AmpLayout& lay, int events, int rank, StagePlan& p, int gm
 	if (gm) {
 		// the waves' FP64 sums [wave][units][columns][4] at the end
 		const uint32_t groups = (p.rowUnits + kGmUnits - 1) / kGmUnits;
-		const int ncs = p.ranks == 1 ? gm_col_sets<1>() : p.ranks == 2 ? gm_col_sets<2>() : gm_col_sets<4>();
+		const int ncs = (p.ranks + 1) / 2;
 		const size_t gmBytes = (size_t)waves * groups * kGmUnits * 4 * ncs * 4 * sizeof(double);
 		p.ldsBytes = std::max(p.ldsBytes, gmBytes);
 	}

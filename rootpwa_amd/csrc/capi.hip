@@ -160,8 +160,6 @@ int configure_grid(rpwa_lik_ctx* c, int slot)
 		return st;
 	}
 	c->nWg[slot] = c->nCu * std::min(wgPerCu, 8);
-	if (const int e = c->tile[slot].events)  // no workgroup without a tile: its empty row would be reduced too
-		c->nWg[slot] = (int)std::min<uint64_t>((uint64_t)c->nWg[slot], std::max<uint64_t>(1, (c->lay.nEvents + e - 1) / e));
 	return RPWA_OK;
 }
 

@@ -410,6 +410,17 @@ int check_mlp(const rpwa_mlp* m, const char* fn)
 	return RPWA_OK;
 }
 
+// parameters p and zero Adam moments.  On the network's own stream: it does not
+// wait for the null stream, so a clear there could run into the next training
+int start_state(rpwa_mlp* m, const float* p)
+{
+	RPWA_HIP_CHECK(hipMemcpyAsync(m->d_p, p, m->nParams * sizeof(float), hipMemcpyHostToDevice, m->stream));
+	RPWA_HIP_CHECK(hipMemsetAsync(m->d_m1, 0, m->nParams * sizeof(float), m->stream));
+	RPWA_HIP_CHECK(hipMemsetAsync(m->d_m2, 0, m->nParams * sizeof(float), m->stream));
+	RPWA_HIP_CHECK(hipStreamSynchronize(m->stream));
+	return RPWA_OK;
+}
+
 int ensure_rows(rpwa_mlp* m, uint32_t rows)
 {
 	if (rows <= m->capRows)
@@ -606,9 +617,8 @@ extern "C" int rpwa_mlp_create(rpwa_mlp** out, int device, uint32_t nIn, uint32_
 	RPWA_HIP_CHECK(hipMalloc(&m->d_m2, m->nParams * sizeof(float)));
 	RPWA_HIP_CHECK(hipMalloc(&m->d_loss, sizeof(float)));
 	RPWA_HIP_CHECK(hipMalloc(&m->d_epoch, sizeof(double)));
-	RPWA_HIP_CHECK(hipMemcpy(m->d_p, p.data(), m->nParams * sizeof(float), hipMemcpyHostToDevice));
-	RPWA_HIP_CHECK(hipMemset(m->d_m1, 0, m->nParams * sizeof(float)));
-	RPWA_HIP_CHECK(hipMemset(m->d_m2, 0, m->nParams * sizeof(float)));
+	if (const int rc = start_state(m.get(), p.data()))
+		return rc;
 	*out = m.release();
 	return RPWA_OK;
 }
@@ -657,10 +667,8 @@ extern "C" int rpwa_mlp_set_params(rpwa_mlp* m, const float* params)
 		return RPWA_ERR_INVALID;
 	}
 	RPWA_HIP_CHECK(hipSetDevice(m->device));
-	RPWA_HIP_CHECK(hipStreamSynchronize(m->stream));
-	RPWA_HIP_CHECK(hipMemcpy(m->d_p, params, m->nParams * sizeof(float), hipMemcpyHostToDevice));
-	RPWA_HIP_CHECK(hipMemset(m->d_m1, 0, m->nParams * sizeof(float)));
-	RPWA_HIP_CHECK(hipMemset(m->d_m2, 0, m->nParams * sizeof(float)));
+	if (const int rc = start_state(m, params))
+		return rc;
 	m->adamStep = 0;
 	return RPWA_OK;
 }

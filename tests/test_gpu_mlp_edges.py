@@ -44,3 +44,23 @@ def test_edges(gpu, shape, rows):
     # relative: 1e-8 / |g| changes by at most the gradient's 10 % error there
     tol = (2.0 ** -24 * (np.abs(want) + 4 * lr) + lr * 0.1 * 1e-8 / np.abs(gref))[big]
     assert np.all(err <= tol)
+
+
+def test_set_params_starts_the_optimiser_anew(gpu):
+    """After setParams a network trains as a new one with these parameters does,
+    bit for bit, however many steps it has taken before: the moments are zero when
+    the next step reads them."""
+    from rootpwa_amd.mlp import MLP
+    rng = np.random.default_rng(11)
+    shape, rows = (775, 512, 2, 176), 128
+    x = rng.normal(size=(rows, shape[0])).astype(np.float32)
+    t = rng.normal(size=(rows, shape[3])).astype(np.float32)
+    fresh = MLP(*shape, seed=4)
+    p = fresh.params()
+    loss = fresh.train(x, t, batchSize=32, epochs=2, lr=1e-3, seed=9)
+    net = MLP(*shape, seed=5)
+    for _ in range(4):
+        net.train(x, t, batchSize=16, epochs=3, lr=1e-2, seed=1)
+        net.setParams(p)
+        assert np.array_equal(net.train(x, t, batchSize=32, epochs=2, lr=1e-3, seed=9), loss)
+        assert np.array_equal(net.params(), fresh.params())

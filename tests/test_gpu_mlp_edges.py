@@ -6,6 +6,8 @@ terms, relative to the largest magnitude: forward 1e-5, gradient 1e-4).  The
 first Adam step moves a parameter by lr g / (|g| + 1e-8): exact to the rounding
 of the parameter (2^-24 relative, and of the quotient, 4 of them) wherever the
 gradient's sign is beyond its own error."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -64,3 +66,26 @@ def test_set_params_starts_the_optimiser_anew(gpu):
         net.setParams(p)
         assert np.array_equal(net.train(x, t, batchSize=32, epochs=2, lr=1e-3, seed=9), loss)
         assert np.array_equal(net.params(), fresh.params())
+
+
+def test_device_memory_held(gpu):
+    """What a network holds after its calls: the activations of the largest call, 4
+    bytes x (nIn + 2 x hidden units + 2 x nOut) a row, and no training set (32 MB of
+    slack for the allocator's granularity)."""
+    from rootpwa_amd.mlp import MLP
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert gpu.lib().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0  # of the library's runtime
+        return a.value
+
+    slack = 32 << 20
+    net = MLP(512, 256, 8, 64, seed=1)
+    start = free()
+    x, t = np.zeros((60000, 512), np.float32), np.zeros((60000, 64), np.float32)
+    net.train(x, t, batchSize=64, epochs=1)  # a set of 138 MB
+    assert start - free() <= slack
+    acts = 60000 * 4 * (512 + 2 * 8 * 256 + 2 * 64)
+    net.forward(x)
+    net.lossGrad(x, t)
+    assert start - free() <= acts + slack

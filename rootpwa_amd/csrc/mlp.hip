@@ -64,8 +64,13 @@ struct GemmArgs {
 	const float* T;         // targets [.][N], row i at T + (tIdx ? tIdx[i] : i) N
 	const uint32_t* tIdx;
 	float scale;            // 2 / (M N)
-	double* tileLoss;       // per workgroup
+	double* tileLoss;       // per tile
+	uint32_t tile0;         // first tile of this launch
 };
+
+// workgroups of one launch: a grid has fewer than 2^32 threads, and an output of
+// 2^31 values (2M rows x 1024) already has 2^23 tiles
+constexpr uint32_t kMaxGrid = 1u << 22;
 
 // 4 consecutive floats at p (aligned to 4 bytes only: rows of any length), zero past `left`
 __device__ __forceinline__ f32x4 load4(const float* p, int left)
@@ -109,7 +114,8 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs a)
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 	const int r = lane & 15, q = lane >> 4;
 	const uint32_t nx = ((uint32_t)a.N + 15) / 16;
-	const int m0 = (int)(blockIdx.x / nx) * 16, n0 = (int)(blockIdx.x % nx) * 16;
+	const uint32_t tile = a.tile0 + blockIdx.x;
+	const int m0 = (int)(tile / nx) * 16, n0 = (int)(tile % nx) * 16;
 	const int m = m0 + r, n = n0 + r;
 	// rows and columns past the edge repeat the last one; their outputs are not stored
 	const int mc = min(m, a.M - 1), nc = min(n, a.N - 1);
@@ -188,7 +194,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs a)
 			__syncthreads();
 		}
 		if (t == 0)
-			a.tileLoss[blockIdx.x] = sq[0];
+			a.tileLoss[tile] = sq[0];
 	}
 }
 
@@ -434,11 +440,14 @@ int ensure_rows(rpwa_mlp* m, uint32_t rows)
 }
 
 template <bool TB, int EPI>
-int gemm(rpwa_mlp* m, const GemmArgs& a)
+int gemm(rpwa_mlp* m, GemmArgs a)
 {
-	const dim3 grid((uint32_t)((a.N + 15) / 16) * (uint32_t)((a.M + 15) / 16));
-	hipLaunchKernelGGL((gemm_kernel<TB, EPI>), grid, dim3(kGemmThreads), 0, m->stream, a);
-	RPWA_HIP_CHECK(hipGetLastError());
+	const uint32_t tiles = (uint32_t)((a.N + 15) / 16) * (uint32_t)((a.M + 15) / 16);
+	for (a.tile0 = 0; a.tile0 < tiles; a.tile0 += std::min(tiles - a.tile0, kMaxGrid)) {
+		hipLaunchKernelGGL((gemm_kernel<TB, EPI>), dim3(std::min(tiles - a.tile0, kMaxGrid)), dim3(kGemmThreads), 0,
+		                   m->stream, a);
+		RPWA_HIP_CHECK(hipGetLastError());
+	}
 	return RPWA_OK;
 }
 

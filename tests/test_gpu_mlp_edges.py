@@ -89,3 +89,16 @@ def test_device_memory_held(gpu):
     net.forward(x)
     net.lossGrad(x, t)
     assert start - free() <= acts + slack
+
+
+def test_more_tiles_than_one_launch(gpu):
+    """An output of more than 2^31 values (2^21 + 16 rows x 1024 hidden units: 2^23 + 64
+    tiles, 17 GB of activations) takes several launches; a row's result does not
+    depend on the rows beside it."""
+    from rootpwa_amd.mlp import MLP
+    rows = (1 << 21) + 16
+    net = MLP(1, 1024, 1, 1, seed=3)
+    x = np.linspace(-3, 3, rows, dtype=np.float32)[:, None]
+    y = net.forward(x)
+    for first in (0, (1 << 16) - 8, (1 << 20) - 8, rows - 16):
+        assert np.array_equal(net.forward(x[first:first + 16]), y[first:first + 16])

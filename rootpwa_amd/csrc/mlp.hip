@@ -36,13 +36,23 @@ __device__ __forceinline__ float gelu_grad(float z)
 // largest one is 64 x 512 x 775 (51 MFLOP, 1.6 MB of weights out of L2): one
 // 32 x 32 tile per wave gave 64 waves, each a chain of 388 dependent load /
 // MFMA steps (111 us).  So a workgroup owns one 16 x 16 tile (128 workgroups
-// there) and its kGemmWaves waves split K: wave w takes the 16-deep K groups w,
-// w + 8, ..., kGemmDeep of them loaded before the first MFMA, and the waves'
+// there) and its up to kGemmWaves waves split K: wave w takes the 16-deep K groups
+// w, w + 8, ..., kGemmDeep of them loaded before the first MFMA, and the waves'
 // sums are added in wave order through LDS (5.0 us on average over the hidden
 // layers; a training step of the 775 - 3 x 512 - 176 network 730 -> 50 us).
+// From kManyTiles tiles on the chip is full and the operands' loads bound a
+// product: there a workgroup takes kRowTiles tiles of 16 rows, whose B is loaded
+// once (gemm_kernel).
 constexpr int kGemmWaves = 8;
 constexpr int kGemmThreads = 64 * kGemmWaves;
 constexpr int kGemmDeep = 4;  // 16-deep K groups in flight per wave
+// Kernels of a forward pass with 1 / kRowTiles tiles per workgroup (with 64 x 64
+// tiles of four waves before K was split): 775 - 3 x 512 - 176 at 1024 rows (2048
+// tiles in a hidden layer) 70 / 53 us (436), at 256 (512 tiles) 26 / 34 (351), at
+// 60000 3.2 / 2.2 ms (4.3); 64 - 2 x 128 - 32 at 4096 rows (2048 tiles) 34 / 18 us
+// (51), at 60000 365 / 113 (165); 300 - 1024 - 60 at 256 rows (1024 tiles) 17 / 20 (177).
+constexpr int kRowTiles = 4;
+constexpr uint32_t kManyTiles = 2048;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -64,12 +74,11 @@ struct GemmArgs {
 	const float* T;         // targets [.][N], row i at T + (tIdx ? tIdx[i] : i) N
 	const uint32_t* tIdx;
 	float scale;            // 2 / (M N)
-	double* tileLoss;       // per tile
-	uint32_t tile0;         // first tile of this launch
+	double* tileLoss;       // per workgroup
+	uint32_t tile0;         // first workgroup of this launch
 };
 
-// workgroups of one launch: a grid has fewer than 2^32 threads, and an output of
-// 2^31 values (2M rows x 1024) already has 2^23 tiles
+// workgroups of one launch: a grid has fewer than 2^32 threads
 constexpr uint32_t kMaxGrid = 1u << 22;
 
 // 4 consecutive floats at p (aligned to 4 bytes only: rows of any length), zero past `left`
@@ -104,32 +113,46 @@ __device__ __forceinline__ void store4(float* p, const f32x4 v, int left)
 	}
 }
 
-// C = A op(B) on one 16 x 16 tile.  MFMA i of a K group takes k = 16 g + 4 q + i
-// in lane quarter q (lane / 16), so a lane's four values are consecutive in a row.
-template <bool TB, int EPI>
+// C = A op(B) on MT tiles of 16 x 16, one below the other; B's values serve all of
+// them, and each tile's sum is the same whatever MT is.  MFMA i of a K group takes
+// k = 16 g + 4 q + i in lane quarter q (lane / 16), so a lane's four values are
+// consecutive in a row.
+template <bool TB, int EPI, int MT>
 __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs a)
 {
-	__shared__ float red[kGemmWaves][256];
-	__shared__ double sq[256];
+	__shared__ float red[kGemmWaves][MT * 256];
+	// fewer waves where K has fewer groups, but with one tile per workgroup (bound by
+	// latency, where the reads of the waves' sums are better known at compile time)
+	const int nThreads = MT > 1 ? (int)blockDim.x : kGemmThreads, nWaves = nThreads / 64;
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 	const int r = lane & 15, q = lane >> 4;
 	const uint32_t nx = ((uint32_t)a.N + 15) / 16;
 	const uint32_t tile = a.tile0 + blockIdx.x;
-	const int m0 = (int)(tile / nx) * 16, n0 = (int)(tile % nx) * 16;
-	const int m = m0 + r, n = n0 + r;
+	const int m0 = (int)(tile / nx) * (16 * MT), n0 = (int)(tile % nx) * 16;
 	// rows and columns past the edge repeat the last one; their outputs are not stored
-	const int mc = min(m, a.M - 1), nc = min(n, a.N - 1);
-	const float* pa = a.A + (size_t)(a.rowIdx ? a.rowIdx[mc] : (uint32_t)mc) * a.lda;
+	const int nc = min(n0 + r, a.N - 1);
+	const float* pa[MT];
+#pragma unroll
+	for (int u = 0; u < MT; ++u) {
+		const int mc = min(m0 + 16 * u + r, a.M - 1);
+		pa[u] = a.A + (size_t)(a.rowIdx ? a.rowIdx[mc] : (uint32_t)mc) * a.lda;
+	}
 	const float* pb = TB ? a.B + (size_t)nc * a.ldb : a.B + nc;
 	const int groups = (a.K + 15) / 16;
-	f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-	for (int g0 = wave; g0 < groups; g0 += kGemmWaves * kGemmDeep) {
-		f32x4 av[kGemmDeep], bv[kGemmDeep];
+	f32x4 acc[MT];
 #pragma unroll
-		for (int d = 0; d < kGemmDeep; ++d) {
+	for (int u = 0; u < MT; ++u)
+		acc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+	constexpr int kDeep = MT > 1 ? 1 : kGemmDeep;
+	for (int g0 = wave; g0 < groups; g0 += kGemmWaves * kDeep) {
+		f32x4 av[kDeep][MT], bv[kDeep];
+#pragma unroll
+		for (int d = 0; d < kDeep; ++d) {
 			const int g = g0 + d * kGemmWaves, k = 16 * g + 4 * q;
 			if (16 * g + 16 <= a.K) {  // the same in every lane
-				av[d] = load4(pa + k, 4);
+#pragma unroll
+				for (int u = 0; u < MT; ++u)
+					av[d][u] = load4(pa[u] + k, 4);
 				if (TB)
 					bv[d] = load4(pb + k, 4);
 				else
@@ -138,7 +161,9 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs a)
 						bv[d][i] = pb[(size_t)(k + i) * a.ldb];
 			} else {  // the last, partial group, and none
 				const int left = a.K - k;
-				av[d] = load4(pa + k, left);
+#pragma unroll
+				for (int u = 0; u < MT; ++u)
+					av[d][u] = load4(pa[u] + k, left);
 				if (TB)
 					bv[d] = load4(pb + k, left);
 				else
@@ -148,23 +173,30 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs a)
 			}
 		}
 #pragma unroll
-		for (int d = 0; d < kGemmDeep; ++d)
+		for (int d = 0; d < kDeep; ++d)
 #pragma unroll
 			for (int i = 0; i < 4; ++i)
-				acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[d][i], bv[d][i], acc, 0, 0, 0);
+#pragma unroll
+				for (int u = 0; u < MT; ++u)
+					acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[d][u][i], bv[d][i], acc[u], 0, 0, 0);
 	}
 	// D[i][j]: column j = lane % 16, row i = 4 (lane / 16) + register
 #pragma unroll
-	for (int v = 0; v < 4; ++v)
-		red[wave][(4 * q + v) * 16 + r] = acc[v];
+	for (int u = 0; u < MT; ++u)
+#pragma unroll
+		for (int v = 0; v < 4; ++v)
+			red[wave][256 * u + (4 * q + v) * 16 + r] = acc[u][v];
 	__syncthreads();
-	const int t = threadIdx.x;
 	double d2 = 0.;
-	if (t < 256) {
-		float s = red[0][t];
+	for (int t = threadIdx.x; t < MT * 256; t += nThreads) {
+		float part[kGemmWaves];
+#pragma unroll
+		for (int w = 0; w < kGemmWaves; ++w)
+			part[w] = w < nWaves ? red[w][t] : 0.f;
+		float s = part[0];
 #pragma unroll
 		for (int w = 1; w < kGemmWaves; ++w)
-			s += red[w][t];
+			s += part[w];
 		const int i = m0 + t / 16, j = n0 + t % 16;
 		if (i < a.M && j < a.N) {
 			const size_t o = (size_t)i * a.N + j;
@@ -175,7 +207,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs a)
 				if (EPI == EPI_LOSS) {
 					const float d = z - a.T[(size_t)(a.tIdx ? a.tIdx[i] : (uint32_t)i) * a.N + j];
 					a.Z[o] = a.scale * d;
-					d2 = (double)d * (double)d;
+					d2 += (double)d * (double)d;
 				} else {
 					a.Z[o] = z;
 				}
@@ -185,15 +217,15 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_kernel(const GemmArgs a)
 		}
 	}
 	if (EPI == EPI_LOSS) {
-		if (t < 256)
-			sq[t] = d2;
+		__shared__ double sq[kGemmThreads];
+		sq[threadIdx.x] = d2;
 		__syncthreads();
-		for (int w = 128; w > 0; w >>= 1) {
-			if (t < w)
-				sq[t] += sq[t + w];
+		for (int w = min(nThreads, MT * 256) / 2; w > 0; w >>= 1) {
+			if ((int)threadIdx.x < w)
+				sq[threadIdx.x] += sq[threadIdx.x + w];
 			__syncthreads();
 		}
-		if (t == 0)
+		if (threadIdx.x == 0)
 			a.tileLoss[tile] = sq[0];
 	}
 }
@@ -350,7 +382,7 @@ struct rpwa_mlp {
 	std::vector<float*> d_Z, d_H;  // per layer: pre-activation, then its gradient [rows][out]; activation (hidden)
 	float* d_x = nullptr;
 	float* d_t = nullptr;
-	double* d_tileLoss = nullptr;  // per 16 x 16 tile of the output: sum of squared errors
+	double* d_tileLoss = nullptr;  // per workgroup of the output's product: sum of squared errors
 	float* d_loss = nullptr;
 	double* d_epoch = nullptr;
 
@@ -439,13 +471,28 @@ int ensure_rows(rpwa_mlp* m, uint32_t rows)
 	return RPWA_OK;
 }
 
+// workgroups of an M x N product
+struct GemmGrid {
+	bool many;
+	uint32_t workgroups;
+	GemmGrid(int M, int N)
+	{
+		const uint32_t rowTiles = ((uint32_t)M + 15) / 16, colTiles = ((uint32_t)N + 15) / 16;
+		many = (uint64_t)rowTiles * colTiles >= kManyTiles;
+		workgroups = (many ? (rowTiles + kRowTiles - 1) / kRowTiles : rowTiles) * colTiles;
+	}
+};
+
 template <bool TB, int EPI>
 int gemm(rpwa_mlp* m, GemmArgs a)
 {
-	const uint32_t tiles = (uint32_t)((a.N + 15) / 16) * (uint32_t)((a.M + 15) / 16);
-	for (a.tile0 = 0; a.tile0 < tiles; a.tile0 += std::min(tiles - a.tile0, kMaxGrid)) {
-		hipLaunchKernelGGL((gemm_kernel<TB, EPI>), dim3(std::min(tiles - a.tile0, kMaxGrid)), dim3(kGemmThreads), 0,
-		                   m->stream, a);
+	const GemmGrid g(a.M, a.N);
+	int waves = g.many ? 1 : kGemmWaves;  // a power of two
+	while (waves < kGemmWaves && waves * 16 < a.K)
+		waves *= 2;
+	for (a.tile0 = 0; a.tile0 < g.workgroups; a.tile0 += std::min(g.workgroups - a.tile0, kMaxGrid)) {
+		hipLaunchKernelGGL(g.many ? (gemm_kernel<TB, EPI, kRowTiles>) : (gemm_kernel<TB, EPI, 1>),
+		                   dim3(std::min(g.workgroups - a.tile0, kMaxGrid)), dim3(64 * waves), 0, m->stream, a);
 		RPWA_HIP_CHECK(hipGetLastError());
 	}
 	return RPWA_OK;
@@ -539,7 +586,7 @@ int backward(rpwa_mlp* m, const Rows& rows, const AdamStep* adam, double* epochS
 	}
 	d.g = m->d_g;
 	d.tileLoss = m->d_tileLoss;
-	d.nTileLoss = ((rows.n + 15) / 16) * (uint32_t)((m->dims[L] + 15) / 16);
+	d.nTileLoss = GemmGrid((int)rows.n, m->dims[L]).workgroups;
 	d.invN = 1. / ((double)rows.n * (double)m->dims[L]);
 	d.loss = m->d_loss;
 	d.epochSum = epochSum;

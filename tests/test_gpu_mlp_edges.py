@@ -17,7 +17,9 @@ pytestmark = pytest.mark.gpu
 
 # (nIn, nHidden, nHiddenLayers, nOut), rows
 EDGES = [((1, 1, 1, 1), 1), ((3, 5, 0, 2), 4), ((15, 16, 1, 17), 16), ((16, 17, 2, 15), 17), ((17, 64, 1, 65), 63),
-         ((31, 33, 16, 3), 64), ((512, 15, 1, 1), 65), ((129, 48, 2, 63), 130), ((775, 64, 1, 176), 64)]
+         ((31, 33, 16, 3), 64), ((512, 15, 1, 1), 65), ((129, 48, 2, 63), 130), ((775, 64, 1, 176), 64),
+         # from 2048 tiles of an output on a workgroup takes four of them
+         ((1, 128, 2, 128), 16 * 256), ((100, 33, 2, 130), 16 * 1024 + 1), ((20, 513, 1, 16), 63 * 16 + 47)]
 
 
 @pytest.mark.parametrize("shape,rows", EDGES)

@@ -9,8 +9,9 @@
  *
  * A network holds on the device its parameters, their gradient and both Adam
  * moments (16 bytes each), the activations of the largest call (rows x 4 bytes x
- * (nIn + 2 x hidden units + 2 x nOut), of a training call's batch only) until it
- * is destroyed; a training call's set is on the device during the call.
+ * (nIn + 2 x hidden units + 2 x nOut), of a training call's batch only) and a
+ * training set of up to 16 MB until it is destroyed; a larger training set is on
+ * the device during its call.
  *
  * Parameters: W_0, b_0, ..., W_L, b_L, float32, W_l row-major [in][out]
  * (y = x W + b).  Host arrays are row-major [rows][features].

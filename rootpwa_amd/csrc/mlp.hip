@@ -366,6 +366,54 @@ uint64_t mix64(uint64_t x)
 
 using namespace rpwa_amd;
 
+namespace {
+
+// Device copy of a training set.  Up to kKeep bytes stay for the next call (30 us of
+// 1500 for an epoch of 1800 x (775 + 176) values, 6.8 MB); a larger one is given back
+// at the end of its call.
+struct TrainingSet {
+	static constexpr size_t kKeep = (size_t)16 << 20;
+	float *x = nullptr, *t = nullptr;
+	uint32_t* idx = nullptr;
+	size_t nX = 0, nT = 0, nIdx = 0;
+	~TrainingSet() { release(); }
+	bool hold(size_t wantX, size_t wantT, size_t wantIdx)
+	{
+		if (wantX <= nX && wantT <= nT && wantIdx <= nIdx)
+			return true;
+		release();
+		if (hipMalloc(&x, wantX * sizeof(float)) != hipSuccess || hipMalloc(&t, wantT * sizeof(float)) != hipSuccess ||
+		    hipMalloc(&idx, wantIdx * sizeof(uint32_t)) != hipSuccess) {
+			release();
+			return false;
+		}
+		nX = wantX, nT = wantT, nIdx = wantIdx;
+		return true;
+	}
+	void release()
+	{
+		(void)hipFree(x);
+		(void)hipFree(t);
+		(void)hipFree(idx);
+		x = t = nullptr;
+		idx = nullptr;
+		nX = nT = nIdx = 0;
+	}
+	// at the end of a call, also a failed one: nothing on the stream uses the set afterwards
+	struct Call {
+		TrainingSet& set;
+		hipStream_t stream;
+		~Call()
+		{
+			(void)hipStreamSynchronize(stream);
+			if (sizeof(float) * (set.nX + set.nT + set.nIdx) > kKeep)
+				set.release();
+		}
+	};
+};
+
+}  // namespace
+
 struct rpwa_mlp {
 	int device = 0;
 	std::vector<int> dims;         // nIn, hidden..., nOut
@@ -385,6 +433,7 @@ struct rpwa_mlp {
 	double* d_tileLoss = nullptr;  // per workgroup of the output's product: sum of squared errors
 	float* d_loss = nullptr;
 	double* d_epoch = nullptr;
+	TrainingSet set;
 
 	~rpwa_mlp() { release(); }
 	void release_acts()
@@ -595,27 +644,6 @@ int backward(rpwa_mlp* m, const Rows& rows, const AdamStep* adam, double* epochS
 	return RPWA_OK;
 }
 
-// Training set of one call, given back at its end: kept for the next call it saved
-// 30 us (of 1500 for an epoch of 1800 x (775 + 176) values)
-struct TrainingSet {
-	hipStream_t stream;
-	float *x = nullptr, *t = nullptr;
-	uint32_t* idx = nullptr;
-	explicit TrainingSet(hipStream_t s) : stream(s) {}
-	~TrainingSet()
-	{
-		(void)hipStreamSynchronize(stream);  // also after a failure: nothing may still use it
-		(void)hipFree(x);
-		(void)hipFree(t);
-		(void)hipFree(idx);
-	}
-	bool allocate(size_t nX, size_t nT, size_t nIdx)
-	{
-		return hipMalloc(&x, nX * sizeof(float)) == hipSuccess && hipMalloc(&t, nT * sizeof(float)) == hipSuccess &&
-		       hipMalloc(&idx, nIdx * sizeof(uint32_t)) == hipSuccess;
-	}
-};
-
 }  // namespace
 
 extern "C" int rpwa_mlp_create(rpwa_mlp** out, int device, uint32_t nIn, uint32_t nHidden, uint32_t nHiddenLayers,
@@ -777,8 +805,9 @@ extern "C" int rpwa_mlp_train(rpwa_mlp* m, const float* x, const float* target, 
 	if (rc != RPWA_OK)
 		return rc;
 	const int nIn = m->dims[0], nOut = m->dims.back();
-	TrainingSet set(m->stream);
-	if (!set.allocate((size_t)nRows * nIn, (size_t)nRows * nOut, nRows)) {
+	TrainingSet& set = m->set;
+	const TrainingSet::Call call{set, m->stream};
+	if (!set.hold((size_t)nRows * nIn, (size_t)nRows * nOut, nRows)) {
 		set_error("rpwa_mlp_train: device allocation failed");
 		return RPWA_ERR_NOMEM;
 	}

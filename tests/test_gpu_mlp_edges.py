@@ -72,8 +72,8 @@ def test_set_params_starts_the_optimiser_anew(gpu):
 
 def test_device_memory_held(gpu):
     """What a network holds after its calls: the activations of the largest call, 4
-    bytes x (nIn + 2 x hidden units + 2 x nOut) a row, and no training set (32 MB of
-    slack for the allocator's granularity)."""
+    bytes x (nIn + 2 x hidden units + 2 x nOut) a row, and a training set of up to
+    16 MB (32 MB of slack, with the allocator's granularity)."""
     from rootpwa_amd.mlp import MLP
 
     def free():

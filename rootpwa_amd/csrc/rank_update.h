@@ -207,17 +207,18 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 					copy16(base, off[i] < last + rowB ? off[i] : last + off[i] % rowB, at + 1024 * (wave + kWaves * i));
 		}
 	};
+	// a weight is used where it is stored, after the products: an earlier use would
+	// wait for the copies in flight as well
 	double wacc = 0., wstage = 0.;
 	auto loadWeight = [&](uint64_t c) {
-		if (WT && tid < CH) {
-			const uint64_t e = c * CH + tid;
-			wstage = e < a.n ? (a.direct ? a.w[e] : 1. / a.w[e]) : 0.;
-		}
+		if (WT && tid < CH)
+			wstage = a.w[min(c * CH + tid, a.n - 1)];
 	};
-	auto storeWeight = [&](int buf) {
+	auto storeWeight = [&](uint64_t c, int buf) {
 		if (WT && tid < CH) {
-			wts[buf * CH + tid] = wstage;
-			wacc += wstage;
+			const double w = c * CH + tid < a.n ? (a.direct ? wstage : 1. / wstage) : 0.;
+			wts[buf * CH + tid] = w;
+			wacc += w;
 		}
 	};
 	// the chunk is in LDS (its copies of all waves have arrived)
@@ -238,7 +239,7 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 	if (c < nChunks) {
 		loadWeight(c);
 		copy(c, 0);
-		storeWeight(0);
+		storeWeight(c, 0);
 		arrive(c, 0);
 	}
 	for (; c < nChunks; c += gridDim.x) {
@@ -250,32 +251,37 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 		const double* xr = lds + buf * P::bufDoubles + (4 * h + lk) * P::ROW + li;
 		const int odd = P::flip * (lk & 1);
 		const double *xe = xr + 16 * odd, *xo = xr - 16 * odd;
-		const double* wr = wts + buf * CH + 4 * h + lk;
-		double v[2][P::NB], w[2] = {1., 1.};
-		read_step<P, G>(xe, xo, v[0]);
-		if (WT)
-			w[0] = wr[0];
-		// steps 2 s + h, operands one step ahead; past the chunk the last is read again
+		if constexpr (WT) {
+			// the multiplies take the matrix core's turns: with the operands a step ahead
+			// they come in front of every step's products and wait there for the other
+			// wave's (1M events x 64 waves: 420 us, in this order 378, unweighted 334)
 #pragma unroll 1
-		for (int s = 0; s < CH / 8; s += 2) {
-			const int s1 = s + 1 < CH / 8 ? s + 1 : s, s2 = s + 2 < CH / 8 ? s + 2 : s;
-			read_step<P, G>(xe + s1 * 8 * P::ROW, xo + s1 * 8 * P::ROW, v[1]);
-			if (WT)
-				w[1] = wr[8 * s1];
-			__builtin_amdgcn_sched_barrier(0);
-			mfma_step<P, G, WT>(v[0], w[0], acc, std::make_integer_sequence<int, NG>{});
-			__builtin_amdgcn_sched_barrier(0);
-			if (s + 1 < CH / 8) {
-				read_step<P, G>(xe + s2 * 8 * P::ROW, xo + s2 * 8 * P::ROW, v[0]);
-				if (WT)
-					w[0] = wr[8 * s2];
+			for (int s = 0; s < CH / 8; ++s) {
+				double v[P::NB];
+				read_step<P, G>(xe + s * 8 * P::ROW, xo + s * 8 * P::ROW, v);
+				mfma_step<P, G, true>(v, wts[buf * CH + 4 * h + lk + 8 * s], acc, std::make_integer_sequence<int, NG>{});
+			}
+		} else {
+			double v[2][P::NB];
+			read_step<P, G>(xe, xo, v[0]);
+			// steps 2 s + h, operands one step ahead; past the chunk the last is read again
+#pragma unroll 1
+			for (int s = 0; s < CH / 8; s += 2) {
+				const int s1 = s + 1 < CH / 8 ? s + 1 : s, s2 = s + 2 < CH / 8 ? s + 2 : s;
+				read_step<P, G>(xe + s1 * 8 * P::ROW, xo + s1 * 8 * P::ROW, v[1]);
 				__builtin_amdgcn_sched_barrier(0);
-				mfma_step<P, G, WT>(v[1], w[1], acc, std::make_integer_sequence<int, NG>{});
+				mfma_step<P, G, false>(v[0], 1., acc, std::make_integer_sequence<int, NG>{});
 				__builtin_amdgcn_sched_barrier(0);
+				if (s + 1 < CH / 8) {
+					read_step<P, G>(xe + s2 * 8 * P::ROW, xo + s2 * 8 * P::ROW, v[0]);
+					__builtin_amdgcn_sched_barrier(0);
+					mfma_step<P, G, false>(v[1], 1., acc, std::make_integer_sequence<int, NG>{});
+					__builtin_amdgcn_sched_barrier(0);
+				}
 			}
 		}
 		if (next < nChunks) {
-			storeWeight(buf ^ 1);
+			storeWeight(next, buf ^ 1);
 			arrive(next, buf ^ 1);
 		} else {
 			__syncthreads();  // LDS is free for the hand-over

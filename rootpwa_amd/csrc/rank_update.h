@@ -77,6 +77,8 @@ struct Tiles {
 	// place of tile t in a row of nT blocks' triangle, or -1 past the row
 	static __device__ __forceinline__ int place(int t, uint32_t winI0, uint32_t winJ0, uint32_t nT)
 	{
+		if (!rect && NI > kMaxWin)  // the only window
+			return t;
 		const uint32_t I = winI0 + row(t), J = rect ? winJ0 + (col(t) - NI) : winI0 + col(t);
 		return J < nT ? (int)(I * nT - I * (I - 1) / 2 + (J - I)) : -1;
 	}
@@ -190,7 +192,10 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 		const uint32_t c = p < 8u * P::nI ? 8 * a.winI0 + p : 8 * a.winJ0 + (p - 8 * P::nI);
 		off[i] = e * a.D * 8 + 16 * min(c, a.D / 2 - 1);
 	}
-	auto copies = [&](int i) { return 64 * (wave + kWaves * i) < CH * P::UNITS; };  // wave-uniform
+	// wave-uniform, and all but the last copy for every wave
+	auto copies = [&](int i) {
+		return 64 * (kWaves - 1 + kWaves * i) < CH * P::UNITS || 64 * (wave + kWaves * i) < CH * P::UNITS;
+	};
 	auto copy = [&](uint64_t c, int buf) {
 		const double* base = a.x + c * CH * a.D;
 		const uint32_t at = lds0 + buf * P::bufDoubles * 8;
@@ -199,12 +204,12 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 			for (int i = 0; i < P::LOADS; ++i)
 				if (copies(i))
 					copy16(base, off[i], at + 1024 * (wave + kWaves * i));
-		} else {  // the last chunk: past the list's end the last event's columns, zeroed afterwards
-			const uint32_t last = (uint32_t)(a.n - c * CH - 1) * a.D * 8, rowB = a.D * 8;
+		} else {  // the last chunk: past the list's end its last unit, zeroed afterwards
+			const uint32_t last = (uint32_t)(a.n - c * CH) * a.D * 8 - 16;
 #pragma unroll
 			for (int i = 0; i < P::LOADS; ++i)
 				if (copies(i))
-					copy16(base, off[i] < last + rowB ? off[i] : last + off[i] % rowB, at + 1024 * (wave + kWaves * i));
+					copy16(base, min(off[i], last), at + 1024 * (wave + kWaves * i));
 		}
 	};
 	// a weight is used where it is stored, after the products: an earlier use would
@@ -292,7 +297,8 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 	// hand-over: the second wave of a pair passes its sums to the first through LDS in
 	// rounds that every wave runs, and the first writes the pair's sum; tiles past the
 	// row are dropped.  v_mfma_f64_16x16x4_f64 leaves D[i][j] in lane j + 16 (i % 4),
-	// register i / 4
+	// register i / 4.  Few branches and little address work a tile: short event lists
+	// are bound by fetching this code (3000 events x 88 waves: 64 -> 56 us a call)
 	double* red = lds + G * P::ROUND * 256;
 	double* out = a.partials + (size_t)blockIdx.x * a.nTiles * 256;
 #pragma unroll
@@ -313,13 +319,16 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 					continue;
 				double* o = out + (size_t)at0 * 256;
 #pragma unroll
-				for (int v = 0; v < 4; ++v) {
-					const int at = (lk + 4 * v) * 16 + li;
-					double val = acc[q][v] + red[((q - r0) * 4 + v) * 64 + lane];
-					if (a.accumulate)
-						val += o[at];
-					o[at] = val;
+				for (int v = 0; v < 4; ++v)
+					acc[q][v] += red[((q - r0) * 4 + v) * 64 + lane];
+				if (a.accumulate) {
+#pragma unroll
+					for (int v = 0; v < 4; ++v)
+						acc[q][v] += o[(lk + 4 * v) * 16 + li];
 				}
+#pragma unroll
+				for (int v = 0; v < 4; ++v)
+					o[(lk + 4 * v) * 16 + li] = acc[q][v];
 			}
 		}
 		__syncthreads();

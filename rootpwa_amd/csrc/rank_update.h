@@ -111,7 +111,7 @@ struct Pass : Tiles<NI, NJ> {
 };
 
 struct Args {
-	const double* x;        // [n][D], 16-byte aligned
+	const double* x;        // [n][D]
 	const double* w;        // weights or null
 	uint64_t n;
 	uint32_t D;             // doubles per row (even)
@@ -122,6 +122,7 @@ struct Args {
 	double* wsum;           // [nWg] sums of the weights, by the first pass; null in the others
 	int accumulate;         // add to the partials of an earlier call
 	int direct;             // weight w[e] instead of 1 / w[e]
+	int odd;                // x is not 16-byte aligned (set by launch)
 };
 
 // 16 bytes per lane of global memory straight into LDS: lane l of the wave
@@ -184,14 +185,15 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 	// the unit a lane copies: number lane + 64 (wave + 8 i) of the chunk's LDS image;
 	// past the row (the last window's padding) the row's last unit, whose products
 	// only reach output elements past the row
-	uint32_t off[P::LOADS];
-#pragma unroll
-	for (int i = 0; i < P::LOADS; ++i) {
-		const uint32_t u = (uint32_t)(lane + 64 * (wave + kWaves * i));
+	auto offset = [&](uint32_t u) {
 		const uint32_t e = u / P::UNITS, p = (u % P::UNITS) ^ (P::flip * 8 * (e & 1));
 		const uint32_t c = p < 8u * P::nI ? 8 * a.winI0 + p : 8 * a.winJ0 + (p - 8 * P::nI);
-		off[i] = e * a.D * 8 + 16 * min(c, a.D / 2 - 1);
-	}
+		return e * a.D * 8 + 16 * min(c, a.D / 2 - 1);
+	};
+	uint32_t off[P::LOADS];
+#pragma unroll
+	for (int i = 0; i < P::LOADS; ++i)
+		off[i] = offset((uint32_t)(lane + 64 * (wave + kWaves * i)));
 	// wave-uniform, and all but the last copy for every wave
 	auto copies = [&](int i) {
 		return 64 * (kWaves - 1 + kWaves * i) < CH * P::UNITS || 64 * (wave + kWaves * i) < CH * P::UNITS;
@@ -199,7 +201,15 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 	auto copy = [&](uint64_t c, int buf) {
 		const double* base = a.x + c * CH * a.D;
 		const uint32_t at = lds0 + buf * P::bufDoubles * 8;
-		if ((c + 1) * CH <= a.n) {
+		if (a.odd) {  // rows at an odd double, through registers: copy16 takes 16-byte aligned units
+			const uint32_t last = (uint32_t)min(a.n - c * CH, (uint64_t)CH) * a.D * 8 - 16;
+#pragma unroll 4
+			for (uint32_t u = tid; u < CH * P::UNITS; u += kThreads) {
+				const double* src = base + min(offset(u), last) / 8;
+				lds[buf * P::bufDoubles + 2 * u] = src[0];
+				lds[buf * P::bufDoubles + 2 * u + 1] = src[1];
+			}
+		} else if ((c + 1) * CH <= a.n) {
 #pragma unroll
 			for (int i = 0; i < P::LOADS; ++i)
 				if (copies(i))
@@ -412,6 +422,7 @@ hipError_t launch(Args a, int nWg, hipStream_t s)
 	a.nT = (a.D + 15) / 16;
 	a.nTiles = a.nT * (a.nT + 1) / 2;
 	const uint32_t nWin = a.nT <= (uint32_t)kOneWin ? 1 : (a.nT + kMaxWin - 1) / kMaxWin;
+	a.odd = reinterpret_cast<uintptr_t>(a.x) % 16 != 0;
 	double* const wsum = a.wsum;
 	for (uint32_t u = 0; u < nWin; ++u)
 		for (uint32_t v = u; v < nWin; ++v) {

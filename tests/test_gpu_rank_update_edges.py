@@ -30,6 +30,23 @@ def test_integral(gpu, waves, events):
     assert H.rel_err(gpu.integral(a, w), ref) <= 1e-12
 
 
+@pytest.mark.parametrize("waves,events", [(1, 3), (9, 65), (88, 64 * 256 + 57), (96, 1000), (137, 300)])
+def test_integral_of_rows_at_an_odd_double(gpu, waves, events):
+    """Device arrays aligned to 8 bytes only give the bits of aligned ones."""
+    rng = np.random.default_rng(waves)
+    a = amplitudes(rng, events, waves)
+    w = rng.uniform(0.5, 2.0, size=events)
+    buf, odd, wbuf = gpu.DeviceBuffer(a.nbytes), gpu.DeviceBuffer(a.nbytes + 16), gpu.DeviceBuffer(w.nbytes)
+    buf.upload(a)
+    odd.upload(np.concatenate([[np.nan], a.view(np.float64).ravel(), [np.nan]]))
+    wbuf.upload(w)
+    for wt in (None, wbuf.address):
+        ref = gpu.integral_device(buf.address, events, waves, wt)
+        assert np.array_equal(gpu.integral_device(odd.address + 8, events, waves, wt), ref)
+        if waves <= 128:
+            assert np.array_equal(gpu.integral_device_noalloc(odd.address + 8, events, waves, wt), ref)
+
+
 def hessian(A, nW, T, flat):
     """[P][P][3], [P], float of pwaLikelihood.cc:697-753 over P = rank 2 wmax amplitudes."""
     rank, wmax = T.shape[0], T.shape[2]

@@ -647,15 +647,26 @@ extern "C" int rpwa_lik_hessian(rpwa_lik_ctx* ctx, const double* prodAmps, uint3
 					gwave[a] = (int)(lay.secOff[sec] + i);
 					valid[a] = (int)(r * lay.rowLen) + gwave[a];
 				}
-		// element (r, c) of the symmetric matrix from its upper-triangle tiles
-		auto element = [](const double* tiles, uint32_t nT, uint32_t r, uint32_t c) {
-			if (r / 16 > c / 16)
-				std::swap(r, c);
-			const uint32_t I = r / 16, J = c / 16;
-			return tiles[(size_t)(I * nT - I * (I - 1) / 2 + (J - I)) * 256 + (r % 16) * 16 + c % 16];
+		// row r of the symmetric matrix from its upper-triangle tiles (products of rows
+		// with themselves: the halves of a diagonal tile are bitwise equal)
+		auto matrix_row = [](const double* tiles, uint32_t nT, uint32_t r, double* out) {
+			const uint32_t I = r / 16, i = r % 16;
+			for (uint32_t J = 0; J < nT; ++J) {
+				const uint32_t lo = std::min(I, J), hi = std::max(I, J);
+				const double* t = tiles + ((size_t)lo * nT - (size_t)lo * (lo - 1) / 2 + (hi - lo)) * 256;
+				for (uint32_t j = 0; j < 16; ++j)
+					out[16 * J + j] = J < I ? t[16 * j + i] : t[16 * i + j];
+			}
 		};
-		auto cd = [&](size_t r, size_t c) { return element(tilesD, nTD, (uint32_t)r, (uint32_t)c); };
-		auto ca = [&](size_t r, size_t c) { return element(tilesA, nTA, (uint32_t)r, (uint32_t)c); };
+		// sum of factor A_a conj(A_b) over the columns of a row: [cA][cA] real and imaginary parts
+		std::vector<double> row0(16 * (size_t)std::max(nTD, nTA)), row1(row0.size());
+		std::vector<double2> Q((size_t)cA * cA);
+		for (uint32_t a = 0; a < cA; ++a) {
+			matrix_row(tilesA, nTA, 2 * a, row0.data());
+			matrix_row(tilesA, nTA, 2 * a + 1, row1.data());
+			for (uint32_t b = 0; b < cA; ++b)
+				Q[(size_t)a * cA + b] = make_double2(row0[2 * b] + row1[2 * b + 1], row1[2 * b] - row0[2 * b + 1]);
+		}
 		std::memset(hessian, 0, ndFull * ndFull * 3 * sizeof(double));
 		for (size_t a = 0; a < ndFull; ++a) {
 			const int va = valid[a];
@@ -663,23 +674,22 @@ extern "C" int rpwa_lik_hessian(rpwa_lik_ctx* ctx, const double* prodAmps, uint3
 				flatTerms[2 * a] = flatTerms[2 * a + 1] = 0.;
 				continue;
 			}
-			const size_t ra = a / (2 * wmax), sa = (a / wmax) % 2;
+			const size_t blockA = a / wmax;  // (rank, sector)
+			matrix_row(tilesD, nTD, 2 * va, row0.data());
+			matrix_row(tilesD, nTD, 2 * va + 1, row1.data());
 			for (size_t b = 0; b < ndFull; ++b) {
 				const int vb = valid[b];
 				if (vb < 0)
 					continue;
-				const size_t rb = b / (2 * wmax), sb = (b / wmax) % 2;
 				double* h = hessian + (a * ndFull + b) * 3;
-				h[0] = cd(2 * va, 2 * vb);
-				h[1] = cd(2 * vb + 1, 2 * va);
-				h[2] = cd(2 * va + 1, 2 * vb + 1);
-				if (ra == rb && sa == sb) {
-					const size_t ga = gwave[a], gb = gwave[b];
-					const double re = ca(2 * ga, 2 * gb) + ca(2 * ga + 1, 2 * gb + 1);
-					const double im = ca(2 * ga + 1, 2 * gb) - ca(2 * ga, 2 * gb + 1);
-					h[0] -= re;
-					h[1] -= im;
-					h[2] -= re;
+				h[0] = row0[2 * vb];
+				h[1] = row0[2 * vb + 1];
+				h[2] = row1[2 * vb + 1];
+				if (b / wmax == blockA) {
+					const double2 q = Q[(size_t)gwave[a] * cA + gwave[b]];
+					h[0] -= q.x;
+					h[1] -= q.y;
+					h[2] -= q.x;
 				}
 			}
 			flatTerms[2 * a] = prodAmpFlat * colD[2 * va];

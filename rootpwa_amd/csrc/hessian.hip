@@ -41,23 +41,24 @@ __device__ __forceinline__ double2 amp_at(const void* amps, uint64_t i)
 
 // factor S of every (rank, sector), factor and sqrt(factor) of every event: with
 // the rows scaled on both sides the products need no weights (FP64 vector
-// multiplies take the matrix core's turns).  16 lanes per event, T [rank][rowLen]
+// multiplies take the matrix core's turns).  L lanes per event, T [rank][rowLen]
 // (zero on padding) from the caches.  Bound by one read of the amplitudes
-// (2M x 88 complex64: 0.38 ms, 3.8 TB/s).
-template <bool MIXED>
+// (2M x 88 complex64: 0.38 ms, 3.8 TB/s), and in narrow rows by the sums over an
+// event's lanes, which are the same for any row length: 4 lanes there.
+template <bool MIXED, uint32_t L>
 __global__ __launch_bounds__(256) void hessian_s_kernel(const void* amps, uint64_t e0, uint64_t n, uint32_t rowLen,
                                                         uint32_t secOff1, uint32_t rank,
                                                         const double2* __restrict__ T, double flat2,
                                                         double2* __restrict__ S, double* __restrict__ wD,
                                                         double* __restrict__ wA)
 {
-	// per group of 16 lanes kE events at a time: their loads are in flight together
+	// per group of L lanes kE events at a time: their loads are in flight together
 	// and share the loads of T
-	constexpr uint32_t L = 16, kR = 2, kE = 4;
+	constexpr uint32_t kR = 2, kE = L / 4;
 	const uint32_t lig = threadIdx.x % L, grp = (threadIdx.x % 64) / L;
 	const uint64_t stride = (uint64_t)gridDim.x * (256 / L * kE);
-	// the loop's bound is the same in a wave's four groups: the sums below take all lanes
-	for (uint64_t first = ((uint64_t)blockIdx.x * 4 + threadIdx.x / 64) * (4 * kE); first < n; first += stride) {
+	// the loop's bound is the same in a wave's groups (16 events): the sums below take all lanes
+	for (uint64_t first = ((uint64_t)blockIdx.x * 4 + threadIdx.x / 64) * 16; first < n; first += stride) {
 		uint64_t row[kE];
 		double sigma[kE];
 #pragma unroll
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(256) void hessian_s_kernel(const void* amps, uint64
 				for (uint32_t i = 0; i < kE; ++i)
 #pragma unroll
 					for (uint32_t r = 0; r < kR; ++r) {
-						const double2 v = make_double2(ek::group_sum<16>(acc[i][r].x), ek::group_sum<16>(acc[i][r].y));
+						const double2 v = make_double2(ek::group_sum<(int)L>(acc[i][r].x), ek::group_sum<(int)L>(acc[i][r].y));
 						if (r == 0 || two)
 							sigma[i] += v.x * v.x + v.y * v.y;
 						if (lig == 4 * i + 2 * r + s)
@@ -127,6 +128,11 @@ __global__ __launch_bounds__(256) void hessian_s_kernel(const void* amps, uint64
 		}
 	}
 }
+
+// Longest row that takes 4 lanes per event.  A call with 4 / 16 lanes, us: 1M events x
+// 4 columns x rank 1 211 / 290, x 24 x rank 2 591 / 646, 300k x 40 x rank 1 281 / 286,
+// x 54 x rank 3 1252 / 1212.
+constexpr uint32_t kNarrow = 40;
 
 // ---------------------------------------------------------------------------
 // Rank-k passes over the windows, tiles and pairs of waves of rank_update.h, with
@@ -365,12 +371,16 @@ __device__ __forceinline__ void pass_body(const PassArgs& a, double* lds, double
 				continue;
 			double* o = out + (size_t)at * 256;
 #pragma unroll
-			for (int v = 0; v < 4; ++v) {
-				double val = acc[q][v] + red[(q * 4 + v) * 64 + lane];
-				if (a.accumulate)
-					val += o[(lk + 4 * v) * 16 + li];
-				o[(lk + 4 * v) * 16 + li] = val;
+			for (int v = 0; v < 4; ++v)
+				acc[q][v] += red[(q * 4 + v) * 64 + lane];
+			if (a.accumulate) {
+#pragma unroll
+				for (int v = 0; v < 4; ++v)
+					acc[q][v] += o[(lk + 4 * v) * 16 + li];
 			}
+#pragma unroll
+			for (int v = 0; v < 4; ++v)
+				o[(lk + 4 * v) * 16 + li] = acc[q][v];
 		}
 	}
 	__syncthreads();  // the hand-over has been read: its area takes the column and weight sums
@@ -582,8 +592,10 @@ extern "C" int rpwa_lik_hessian(rpwa_lik_ctx* ctx, const double* prodAmps, uint3
 		for (uint64_t e0 = 0; e == hipSuccess && e0 < lay.nEvents; e0 += cn) {
 			const uint64_t n = std::min<uint64_t>(cn, lay.nEvents - e0);
 			const uint32_t nb = (uint32_t)std::min<uint64_t>((n + 63) / 64, 8ull * nWg);
-			hipLaunchKernelGGL(mixed ? hessian_s_kernel<true> : hessian_s_kernel<false>, dim3(nb), dim3(256), 0, s,
-			                   ctx->d_amps, e0, n, lay.rowLen, lay.secOff[1], rank,
+			const bool narrow = lay.rowLen <= kNarrow;
+			hipLaunchKernelGGL(mixed ? (narrow ? hessian_s_kernel<true, 4> : hessian_s_kernel<true, 16>)
+			                         : (narrow ? hessian_s_kernel<false, 4> : hessian_s_kernel<false, 16>),
+			                   dim3(nb), dim3(256), 0, s, ctx->d_amps, e0, n, lay.rowLen, lay.secOff[1], rank,
 			                   reinterpret_cast<const double2*>(at(offT)), prodAmpFlat * prodAmpFlat,
 			                   reinterpret_cast<double2*>(work.buf), at(offWD), at(offWA));
 			e = hipGetLastError();

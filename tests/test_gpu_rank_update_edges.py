@@ -73,7 +73,8 @@ def hessian(A, nW, T, flat):
 
 @pytest.mark.parametrize("nW,rank,events", [((0, 1), 1, 1), ((7, 0), 1, 63), ((3, 5), 2, 65), ((2, 3), 5, 40),
                                             ((8, 80), 1, 56), ((0, 96), 1, 300), ((1, 103), 1, 64),
-                                            ((0, 136), 1, 129), ((13, 40), 3, 1000), ((5, 37), 4, 700), ((8, 80), 2, 64 * 256 * 2 + 9)])
+                                            ((0, 136), 1, 129), ((13, 40), 3, 1000), ((5, 37), 4, 700), ((3, 36), 3, 130),
+                                            ((8, 80), 2, 64 * 256 * 2 + 9)])
 @pytest.mark.parametrize("prec", [0, 1], ids=["fp64", "mixed"])
 def test_hessian(gpu, nW, rank, events, prec):
     rng = np.random.default_rng(sum(nW) + rank)

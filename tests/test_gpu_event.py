@@ -8,9 +8,11 @@ from tests import helpers as H
 
 pytestmark = pytest.mark.gpu
 
-# (refl -1 waves, refl +1 waves), rank; (30, 170) makes the LDS-staged kernel use 16-event tiles
+# (refl -1 waves, refl +1 waves), rank; (30, 170) makes the LDS-staged kernel use 16-event tiles.
+# Ranks 3 and 4 with one to three unit groups of the MFMA gradient, T in the kernel arguments
+# and (more than 64 and 48 columns) in memory
 SHAPES = [((0, 16), 1), ((3, 5), 2), ((8, 80), 2), ((7, 34), 2), ((1, 1), 1), ((5, 0), 1), ((4, 9), 3),
-          ((30, 170), 2)]
+          ((30, 170), 2), ((13, 40), 3), ((8, 80), 3), ((30, 170), 3), ((4, 9), 4), ((13, 40), 4), ((8, 80), 4)]
 
 
 @pytest.fixture(scope="module", params=SHAPES, ids=lambda p: "W%d+%d_r%d" % (p[0][0], p[0][1], p[1]))
@@ -136,6 +138,26 @@ def test_stage_gradient_on_mfma(gpu, case, events, variant):
         assert fv == f and dfv == df
     assert abs(fv - f) <= 1e-12 * abs(f)
     assert np.max(np.abs(d - dv)) <= 1e-6 * np.max(np.abs(dv))
+    ctx.close()
+
+
+@pytest.mark.parametrize("rank", [1, 2, 3, 4])
+def test_stage_gradient_of_four_unit_groups(gpu, rank):
+    """Rows of 49 to 64 units (9 + 100 waves): tiles of 32 events."""
+    nW = (9, 100)
+    ds = H.dataset(nW, rank, nData=777, nMC=3000, seed=20 + rank)
+    L = H.oracle_likelihood(ds)
+    ctx = gpu.LikelihoodContext(0, 1)
+    ctx.load(H.normalised_amps(L), nW)
+    prod = H.random_prod(np.random.default_rng(31), rank, nW, 0.9)
+    d_ref, df_ref = L.event_deriv(prod, 0.1)
+    for variant in (0, 1):
+        ctx.set_stage_variant(32, variant)
+        assert ctx.kernel_variant(rank)["gradient_mfma"] == variant
+        f, d, df = ctx.fdf(prod, 0.1)
+        assert abs(f - L.event_loglik(prod, 0.1)) <= 1e-6 * abs(f)
+        assert H.rel_err(d, d_ref) <= 1e-5
+        assert abs(df - df_ref) <= 1e-5 * abs(df_ref)
     ctx.close()
 
 

@@ -12,7 +12,11 @@ from tests import test_gpu_batch as TB
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("waves,starts", [(1, 1), (3, 8), (7, 9), (8, 16), (9, 17), (16, 24), (23, 25), (40, 33), (88, 64)])
+@pytest.mark.parametrize("waves,starts", [(1, 1), (3, 8), (7, 9), (8, 16), (9, 17), (16, 24), (23, 25), (40, 33), (88, 64),
+                                          # every swizzle of the rows (padded waves / 8 odd, even, a multiple of
+                                          # 4) in both kinds of unit, up to the most waves
+                                          (25, 12), (32, 57), (48, 45), (56, 20), (64, 16), (72, 10), (80, 56),
+                                          (89, 13), (96, 64)])
 def test_edges(gpu, waves, starts):
     bins = TB.make_bins(waves, [31, 32, 33, 1025], seed=320 + waves)
     par = TB.fp32_params(np.random.default_rng(waves), len(bins), starts, 2 * waves, 2.0)

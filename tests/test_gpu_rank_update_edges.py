@@ -92,3 +92,23 @@ def test_hessian(gpu, nW, rank, events, prec):
     assert H.rel_err(h, rh) <= 1e-12
     assert H.rel_err(ft, rft) <= 1e-12
     assert abs(hf - rhf) <= 1e-12 * abs(rhf) * 10  # a difference of two sums
+
+
+def test_hessian_in_pieces(gpu):
+    """An event list of more than 8 GiB of S (rank 100: 3216 bytes an event) is
+    summed in pieces that add to each other.  Reference: the sum of two lists of
+    one piece each."""
+    rank, nW = 100, (1, 1)
+    piece = (8 << 30) // (32 * rank + 16)
+    N, first = piece + 300_001, piece - 100_003
+    rng = np.random.default_rng(3)
+    A = rng.normal(size=(N, 2)) + 1j * rng.normal(size=(N, 2))
+    T = (rng.normal(size=(rank, 2, 1)) + 1j * rng.normal(size=(rank, 2, 1)))
+    out = []
+    for a in (A, A[:first], A[first:]):
+        ctx = gpu.LikelihoodContext(0, 0)
+        ctx.load(a, nW)
+        out.append(ctx.hessian(T, 0.7))
+        ctx.close()
+    for whole, x, y in zip(*out):
+        assert H.rel_err(whole, x + y) <= 1e-12

@@ -104,3 +104,54 @@ def test_more_tiles_than_one_launch(gpu):
     y = net.forward(x)
     for first in (0, (1 << 16) - 8, (1 << 20) - 8, rows - 16):
         assert np.array_equal(net.forward(x[first:first + 16]), y[first:first + 16])
+
+
+def _mix64(x):
+    m = (1 << 64) - 1
+    x = (x + 0x9E3779B97F4A7C15) & m
+    x = ((x ^ (x >> 30)) * 0xBF58476D1CE4E5B9) & m
+    x = ((x ^ (x >> 27)) * 0x94D049BB133111EB) & m
+    return x ^ (x >> 31)
+
+
+def _adam(p, state, shape, x, t, batch, epochs, lr, seed):
+    """FP64 Adam over the documented shuffle; state: both moments and the step count."""
+    m1, m2, k = state
+    losses = []
+    for epoch in range(epochs):
+        perm = list(range(len(x)))
+        for i in range(len(x) - 1, 0, -1):
+            j = _mix64(seed ^ _mix64((epoch << 32) + i)) % (i + 1)
+            perm[i], perm[j] = perm[j], perm[i]
+        total = 0.0
+        for b in range(len(x) // batch):
+            at = perm[b * batch:(b + 1) * batch]
+            loss, g = M.loss_grad(M.unpack(p, *shape), x[at], t[at])
+            k += 1
+            m1, m2 = 0.9 * m1 + 0.1 * g, 0.999 * m2 + 0.001 * g * g
+            p = p - lr * (m1 / (1 - 0.9 ** k)) / (np.sqrt(m2 / (1 - 0.999 ** k)) + 1e-8)
+            total += loss
+        losses.append(total / (len(x) // batch))
+    return p, (m1, m2, k), losses
+
+
+@pytest.mark.parametrize("shape", [(13, 24, 2, 5), (40, 33, 1, 70)])
+def test_training_steps(gpu, shape):
+    """Batches smaller than a set that is no multiple of them, several epochs, and a
+    second call that goes on with the optimiser's state, against FP64 Adam.  Of the
+    parameters' whole change (2-norm) FP64 Adam's differs by 6e-5 with errors of
+    1e-6 of the largest component in every gradient (the FP32 sums' are below), and
+    by 0.1 where the second call forgets the moments; allowed 5e-4.  Losses 1e-5."""
+    from rootpwa_amd.mlp import MLP
+    rng = np.random.default_rng(1)
+    net = MLP(*shape, seed=1)
+    p0 = (rng.normal(size=net.nParams()) / np.sqrt(24)).astype(np.float32)
+    x = rng.normal(size=(150, shape[0])).astype(np.float32)
+    t = rng.normal(size=(150, shape[3])).astype(np.float32)
+    net.setParams(p0)
+    p, state = p0.astype(np.float64), (0.0, 0.0, 0)
+    for epochs, seed in ((3, 5), (2, 6)):
+        loss = net.train(x, t, batchSize=32, epochs=epochs, lr=1e-3, seed=seed)
+        p, state, ref = _adam(p, state, shape, x.astype(np.float64), t.astype(np.float64), 32, epochs, 1e-3, seed)
+        assert np.max(np.abs(loss / np.array(ref) - 1)) <= 1e-5
+        assert np.linalg.norm(net.params() - p) <= 5e-4 * np.linalg.norm(p - p0)

@@ -68,17 +68,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));  // one 16-byte unit
 
 // G phase: consecutive units of one sector handled by one thread (the
 // weights u of an event are read once for all of them)
-template <bool MIXED, int R>
-constexpr int group_units() { return (MIXED ? 2 : 1) * R <= 2 ? 4 : 2; }
+constexpr int group_units(bool mixed, int R) { return (mixed ? 2 : 1) * R <= 2 ? 4 : 2; }
 // LDS exchange area: complex values per event (2 sectors x R ranks, plus one
 // so that lanes reading consecutive events hit distinct banks)
-template <int R>
-constexpr int part_stride() { return 2 * R + 1; }
+constexpr int part_stride(int R) { return 2 * R + 1; }
 typedef const __attribute__((address_space(4))) double cdouble;
 
 // MFMA gradient: column sets of four (u_re, u_im per rank) and unit groups of 16
-template <int R>
-constexpr int gm_col_sets() { return (2 * R + 3) / 4; }
+constexpr int gm_col_sets(int R) { return (2 * R + 3) / 4; }
 constexpr int kGmUnits = 16;     // units per MFMA (one per block)
 constexpr int kGmMaxGroups = 4;  // rows of at most 64 units
 typedef float gm_f4 __attribute__((ext_vector_type(4)));
@@ -145,7 +142,7 @@ __device__ __forceinline__ void s_phase(const StageArgs& a, const f32x4* stage, 
                                         double2 (&S)[2][R])
 {
 	constexpr int P = MIXED ? 2 : 1;
-	constexpr int PS = part_stride<R>();
+	constexpr int PS = part_stride(R);
 #pragma unroll
 	for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -199,7 +196,7 @@ __device__ __forceinline__ void sigma_phase(const StageArgs& a, const double2* p
                                             uint32_t tile, double2 (&S)[2][R], double& mant, int& expo,
                                             double& wsum)
 {
-	constexpr int PS = part_stride<R>();
+	constexpr int PS = part_stride(R);
 	if (!(E == 64 || lane < E))
 		return;
 #pragma unroll
@@ -250,7 +247,7 @@ __device__ __forceinline__ void sigma_phase(const StageArgs& a, const double2* p
 	}
 	if (GM) {
 		// FP32 u by [sector][column][event], columns (re, im) per rank, zero past 2R
-		constexpr int NCOL = 4 * gm_col_sets<R>();
+		constexpr int NCOL = 4 * gm_col_sets(R);
 		float* uf = reinterpret_cast<float*>(uOut);
 #pragma unroll
 		for (int s = 0; s < 2; ++s) {
@@ -279,9 +276,9 @@ __device__ __forceinline__ void sigma_phase(const StageArgs& a, const double2* p
 template <int R, int E, int NG>
 __device__ __forceinline__ void gm_phase(const StageArgs& a, const f32x4* stage, const float* uf, int wid,
                                          const uint32_t (&aOff)[NG], const uint32_t (&bOff)[NG],
-                                         double (&GD)[NG][gm_col_sets<R>()][4])
+                                         double (&GD)[NG][gm_col_sets(R)][4])
 {
-	constexpr int NCS = gm_col_sets<R>();
+	constexpr int NCS = gm_col_sets(R);
 	constexpr int EW = E / 4;
 	if (a.mode == STAGE_SIGMA)
 		return;
@@ -327,11 +324,11 @@ __device__ __forceinline__ void gm_phase(const StageArgs& a, const f32x4* stage,
 template <bool MIXED, int R, int E>
 __device__ __forceinline__ void g_phase(const StageArgs& a, const f32x4* stage, const double2* uIn, bool gOn,
                                         uint32_t gU0, uint32_t gSub, int gSec,
-                                        double2 (&G)[group_units<MIXED, R>()][MIXED ? 2 : 1][R])
+                                        double2 (&G)[group_units(MIXED, R)][MIXED ? 2 : 1][R])
 {
 	constexpr int P = MIXED ? 2 : 1;
-	constexpr int UG = group_units<MIXED, R>();
-	constexpr int PS = part_stride<R>();
+	constexpr int UG = group_units(MIXED, R);
+	constexpr int PS = part_stride(R);
 	if (!gOn || a.mode == STAGE_SIGMA)
 		return;
 	// The slots of a group are consecutive units, read at fixed offsets from one
@@ -435,10 +432,10 @@ __device__ __forceinline__ void write_log_sums_all_waves(const StageArgs& a, dou
 // u conj(x) = (u_re x_re + u_im x_im) + i (u_im x_re - u_re x_im) ----
 template <int R, int E, int NG, int NT, bool ALLW = false>
 __device__ __forceinline__ void write_partial_row_gm(const StageArgs& a, f32x4* smem, int tid, int lane, int wid,
-                                                     const double (&GD)[NG][gm_col_sets<R>()][4], double mant,
+                                                     const double (&GD)[NG][gm_col_sets(R)][4], double mant,
                                                      int expo, double wsum, double (*lsum)[3] = nullptr)
 {
-	constexpr int NCS = gm_col_sets<R>();
+	constexpr int NCS = gm_col_sets(R);
 	constexpr int NCOL = 4 * NCS;
 	constexpr int UN = kGmUnits * NG;  // units per wave in the buffer
 	lds_barrier();
@@ -493,11 +490,11 @@ __device__ __forceinline__ void write_partial_row_gm(const StageArgs& a, f32x4* 
 template <bool MIXED, int R, int E, int NT>
 __device__ __forceinline__ void write_partial_row(const StageArgs& a, f32x4* smem, int tid, int lane, int wid, bool gOn,
                                                   uint32_t gU0, uint32_t gEnd, uint32_t gSub,
-                                                  double2 (&G)[group_units<MIXED, R>()][MIXED ? 2 : 1][R],
+                                                  double2 (&G)[group_units(MIXED, R)][MIXED ? 2 : 1][R],
                                                   double mant, int expo, double wsum)
 {
 	constexpr int P = MIXED ? 2 : 1;
-	constexpr int UG = group_units<MIXED, R>();
+	constexpr int UG = group_units(MIXED, R);
 	lds_barrier();
 	double2* gbuf = reinterpret_cast<double2*>(smem);  // [gSubs][rowUnits][P][R]
 	if (gOn) {
@@ -646,10 +643,10 @@ template <bool MIXED, int R, int E, int NG>
 __global__ __launch_bounds__(kThreads, 2) void stage_kernel(StageArgs a)
 {
 	constexpr int P = MIXED ? 2 : 1;  // complex values per 16-byte unit
-	constexpr int UG = group_units<MIXED, R>();
+	constexpr int UG = group_units(MIXED, R);
 	constexpr bool GM = NG > 0;
 	constexpr int NGX = GM ? NG : 1;
-	constexpr int NCS = gm_col_sets<R>();
+	constexpr int NCS = gm_col_sets(R);
 	static_assert(!GM || MIXED, "the MFMA gradient needs complex64 amplitudes");
 	extern __shared__ f32x4 smem[];
 	f32x4* stage = smem;  // [E][rowUnitsP] units, then the dump unit
@@ -1106,7 +1103,7 @@ bool stage_plan(const AmpLayout& lay, int events, int rank, StagePlan& p, int gm
 	p.rowUnitsP = p.rowUnits | 1u;
 	p.ranks = stage_rank_cap(rank);
 	const bool mixed = lay.precision == RPWA_PREC_MIXED;
-	const uint32_t ug = (uint32_t)((mixed ? 2 : 1) * p.ranks <= 2 ? 4 : 2);  // group_units
+	const uint32_t ug = (uint32_t)group_units(mixed, p.ranks);
 	const uint32_t secUnit = lay.secOff[1] * bpc / 16u;
 	p.gGroups0 = (secUnit + ug - 1) / ug;
 	p.gGroups = p.gGroups0 + (p.rowUnits - secUnit + ug - 1) / ug;
@@ -1114,7 +1111,7 @@ bool stage_plan(const AmpLayout& lay, int events, int rank, StagePlan& p, int gm
 		return false;
 	p.gSubs = (uint32_t)threads / p.gGroups;
 	p.stageBytes = ((uint32_t)events * p.rowUnitsP + 1u) * 16u;
-	const int ps = 2 * p.ranks + 1;  // part_stride
+	const int ps = part_stride(p.ranks);
 	// S partials of waves 1..3 (u replaces wave 1's)
 	const size_t partBytes = (size_t)(waves - 1) * events * ps * sizeof(double2);
 	const size_t endBytes = (size_t)p.gSubs * p.rowUnits * P * p.ranks * sizeof(double2) +
@@ -1123,7 +1120,7 @@ bool stage_plan(const AmpLayout& lay, int events, int rank, StagePlan& p, int gm
 	if (gm) {
 		// the waves' FP64 sums [wave][units][columns][4] at the end
 		const uint32_t groups = (p.rowUnits + kGmUnits - 1) / kGmUnits;
-		const int ncs = (p.ranks + 1) / 2;
+		const int ncs = gm_col_sets(p.ranks);
 		const size_t gmBytes = (size_t)waves * groups * kGmUnits * 4 * ncs * 4 * sizeof(double);
 		p.ldsBytes = std::max(p.ldsBytes, gmBytes);
 	}

@@ -20,6 +20,8 @@ COMMON = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I", os.path.join(ROOT, "include"), "-I", CSRC,
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
+    # the copies straight into LDS list m0, a reserved register, as clobbered
+    "-Wno-inline-asm",
 ]
 
 

@@ -3,7 +3,7 @@
 // One evaluation of all fits is four kernels, captured once in a hipGraph and
 // replayed for every L-BFGS iteration:
 //   batch_event_kernel   persistent workgroups; each takes work units (bin,
-//                        chunk of 32 tiles of 32 events, group of 16 starts)
+//                        chunk of 32 tiles of 32 events, up to 32 starts)
 //                        and computes, tile by tile, S = A T (FP32 MFMA),
 //                        sigma, ln sigma (FP64) and G += A^H (S / sigma) (FP32
 //                        MFMA), writing one partial per unit;
@@ -1137,7 +1137,7 @@ using namespace rpwa_amd;
 
 struct rpwa_batch {
 	int device = 0;
-	uint32_t W = 0, Wp = 0, rowLen = 0, NT = 0, nStarts = 0, P = 0;
+	uint32_t W = 0, Wp = 0, rowLen = 0, nStarts = 0, P = 0;
 	hipStream_t stream = nullptr;
 	hipEvent_t ev0 = nullptr, ev1 = nullptr;
 	int nCu = 0;
@@ -1416,7 +1416,6 @@ extern "C" int rpwa_batch_create(rpwa_batch** out, int device, uint32_t nmbWaves
 	b->W = nmbWaves;
 	b->Wp = (nmbWaves + 7) / 8 * 8;
 	b->rowLen = 2 * b->Wp;
-	b->NT = (b->rowLen + 31) / 32;
 	b->nStarts = nmbStarts;
 	b->P = 2 * nmbWaves;
 	RPWA_HIP_CHECK(hipSetDevice(device));

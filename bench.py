@@ -265,9 +265,10 @@ def main():
     def timed(L, label):
         ctx = L.gpuContext()
         # HIP events bound to the launches of every TIMING_PERIOD-th evaluation in the timed
-        # region: the kernel durations of the roofline (events on every launch add ~15 us of
-        # host time to each evaluation; the bench reports that rate as well)
-        ctx.set_timing(TIMING_PERIOD)
+        # region (at least one of a shorter loop): the kernel durations of the roofline (events
+        # on every launch add ~15 us of host time to each evaluation; the bench reports that
+        # rate as well)
+        ctx.set_timing(min(TIMING_PERIOD, args.steps))
         for _ in range(args.warmup):
             L.FdF(par)
         capi.synchronize()
@@ -433,7 +434,7 @@ def main():
         # launches of every TIMING_PERIOD-th evaluation; the same FdF loop with timing off
         # (the library's default: no events, completion read from the reduction's flag)
         # and with events on every evaluation
-        "kernel_timing": {"every_nth_evaluation": TIMING_PERIOD,
+        "kernel_timing": {"every_nth_evaluation": min(TIMING_PERIOD, args.steps),
                           "timed_launches": {"mixed": r_mix["timed_launches"], "fp64": r_64["timed_launches"]}},
         "without_kernel_events": {"mixed_evals_per_s": r_mix["rate_without_events"],
                                   "fp64_evals_per_s": r_64["rate_without_events"]},

@@ -17,8 +17,8 @@
 // adds to the products instead of running beside them (5M events x 88 waves:
 // products alone 2.3 ms, copy alone 1.3 ms, both 2.7 to 3.4 ms), so a chunk is
 // copied by global_load_lds, whose addresses are a scalar base and lane offsets
-// that stay the same for every chunk: 2.73 -> 2.61 ms (67 TFLOP/s).  Weights cost
-// FP64 multiplies of the operands (51 TFLOP/s).
+// that stay the same for every chunk: a call 2.73 -> 2.59 ms (65 TFLOP/s of issued
+// products).  Weights cost FP64 multiplies of the operands (2M x 88: 1.05 -> 1.11 ms).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -134,6 +134,13 @@ __device__ __forceinline__ void copy16(const double* base, uint32_t off, uint32_
 	             : "memory", "m0");
 }
 
+// 4 bytes per lane, for rows that are not 16-byte aligned: lane l writes base + 4 l
+__device__ __forceinline__ void copy4(const double* base, uint32_t off, uint32_t ldsBase)
+{
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(ldsBase), "v"(off), "s"(base)
+	             : "memory", "m0");
+}
+
 template <class P, int T>
 struct TileRC {
 	static constexpr int r = P::row(T), c = P::col(T);
@@ -201,14 +208,11 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 	auto copy = [&](uint64_t c, int buf) {
 		const double* base = a.x + c * CH * a.D;
 		const uint32_t at = lds0 + buf * P::bufDoubles * 8;
-		if (a.odd) {  // rows at an odd double, through registers: copy16 takes 16-byte aligned units
+		if (a.odd) {  // 16 units at a time, past the list's end its last unit
 			const uint32_t last = (uint32_t)min(a.n - c * CH, (uint64_t)CH) * a.D * 8 - 16;
-#pragma unroll 4
-			for (uint32_t u = tid; u < CH * P::UNITS; u += kThreads) {
-				const double* src = base + min(offset(u), last) / 8;
-				lds[buf * P::bufDoubles + 2 * u] = src[0];
-				lds[buf * P::bufDoubles + 2 * u + 1] = src[1];
-			}
+#pragma unroll 1
+			for (int i = wave; i < CH * P::UNITS / 16; i += kWaves)
+				copy4(base, min(offset(16 * i + lane / 4), last) + 4 * (lane % 4), at + 256 * i);
 		} else if ((c + 1) * CH <= a.n) {
 #pragma unroll
 			for (int i = 0; i < P::LOADS; ++i)
@@ -269,7 +273,7 @@ __device__ __forceinline__ void body(const Args& a, double* lds, double* wsh)
 		if constexpr (WT) {
 			// the multiplies take the matrix core's turns: with the operands a step ahead
 			// they come in front of every step's products and wait there for the other
-			// wave's (1M events x 64 waves: 420 us, in this order 378, unweighted 334)
+			// wave's (1M events x 64 waves: 420 us, in this order 380, unweighted 330)
 #pragma unroll 1
 			for (int s = 0; s < CH / 8; ++s) {
 				double v[P::NB];

@@ -11,7 +11,7 @@
 // the stored amplitudes while they copy a chunk of events into LDS, so that no
 // row array goes through memory.  The flat wave's terms are column sums of factor2
 // d, taken by the threads that form d, and sums of the factors.
-// 2M events x 88 waves x rank 2, complex64 amplitudes: 9.98 -> 7.28 ms; before, a
+// 2M events x 88 waves x rank 2, complex64 amplitudes: 9.98 -> 7.16 ms; before, a
 // kernel wrote the rows (8.5 GB, 2.3 ms) and weighted passes read them (7.1 ms).
 #include "event_kernel.h"
 #include "hessian_pass.h"

@@ -3,7 +3,7 @@
 // copied: loads of a chunk's amplitudes and S are in flight beside the products of
 // the chunk before it, the entries are stored to LDS between the later products.
 // Bound by FP64 MFMA (64 cycles per tile and step) plus the vector work of forming
-// the rows, which takes the same unit: 41 to 53 TFLOP/s at 28 to 66 tiles per pass; a
+// the rows, which takes the same unit: 42 to 54 TFLOP/s at 28 to 66 tiles per pass; a
 // pass with more tiles forms fewer entries per product.
 #pragma once
 
